@@ -14,35 +14,19 @@
 // The weight gradient dWk[tap][o][i] = sum_vox dY[vox][o] X[vox+s(tap)][i] is
 // a second kernel that reduces over voxels (split over blocks, FP32 atomics).
 //
+// The forward pass of inputs in multiples of 32 channels marches along z
+// (gm_conv_march.hip); the kernels here take the rest: 16-channel inputs, the
+// split sums of volumes with few tiles, unaligned or very large operands.
+//
 // Tiles: a block of 4 waves computes 64 x 64 outputs; each wave a 32 x 32
 // quarter as 2 x 2 MFMA tiles of 16 x 16 (k_conv_fwd32 on large volumes with
 // up to 32 outputs: waves of 64 voxels x 32 outputs); K advances through LDS one tap and
 // 32 input channels at a time (k_conv_fwd32, software-pipelined) or, for 16
 // input channels, 16 at a time (k_conv_fwd).
 
-#include <hip/hip_runtime.h>
-#include <stdint.h>
-
-#include "gm_internal.h"
+#include "gm_conv.h"
 
 namespace gm {
-
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    // round to nearest even (finite inputs)
-    const uint32_t u = __float_as_uint(f);
-    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
-
-struct ConvDims {
-    int nb, D, H, W;  // batch and spatial extent
-    int ci, co;       // channels (multiples of 16)
-    int64_t nvox;     // nb * D * H * W
-};
 
 // (x, y, z) of a voxel, decoded once per thread (32-bit divisions while the
 // volume has fewer than 2^32 voxels)
@@ -723,6 +707,10 @@ static void launch_plan(const FwdPlan& p, const ConvDims& c, const uint16_t* X,
 void launch_conv_fwd(const int32_t* shape, const uint16_t* X, const uint16_t* Wk,
                      const float* bias, int relu, float* Y, uint16_t* Ybf, hipStream_t s) {
     const ConvDims c = dims(shape);
+    if (conv_march_ok(c, X, Wk, Y, Ybf)) {
+        launch_conv_march(c, X, Wk, bias, relu, Y, Ybf, s);
+        return;
+    }
     const bool al16 = (((uintptr_t)X | (uintptr_t)Wk) & 15) == 0;
     launch_plan(plan_fwd(c, al16), c, X, Wk, bias, relu, Y, Ybf, nullptr, s);
 }
@@ -741,7 +729,11 @@ void launch_conv_fwd_ws(const int32_t* shape, const uint16_t* X, const uint16_t*
     const FwdPlan p = plan_fwd(c, al16);
     const bool split = p.fwd32 && p.splits > 1 && ws &&
                        ws_bytes >= (int64_t)p.splits * c.nvox * c.co * 4;
-    launch_plan(p, c, X, Wk, bias, relu, Y, Ybf, split ? (float*)ws : nullptr, s);
+    if (!split) {
+        launch_conv_fwd(shape, X, Wk, bias, relu, Y, Ybf, s);
+        return;
+    }
+    launch_plan(p, c, X, Wk, bias, relu, Y, Ybf, (float*)ws, s);
 }
 
 void launch_conv_wflip(int ci, int co, const uint16_t* Wk, uint16_t* Wt, hipStream_t s) {

@@ -89,6 +89,49 @@ def test_conv_gradients(S, shape):
     assert _rel(dW.cpu().numpy() - base, ref) < 1e-5
 
 
+# the marching kernel's edges: partial tiles in x, y and z, 8- and 16-wide
+# tiles, output counts off its tiles, one plane, one voxel, volumes cut into z
+# segments, channel stages up to the LDS limit and past it (352: the
+# tap-by-tap kernel), and few tiles (the split sum of the forward pass)
+MARCH = [(1, 3, 19, 33, 32, 48), (2, 5, 17, 8, 64, 96), (1, 33, 9, 40, 32, 80),
+         (1, 1, 1, 1, 32, 16), (3, 1, 30, 23, 64, 32), (1, 7, 34, 17, 160, 32),
+         (2, 4, 12, 20, 256, 64), (1, 2, 9, 16, 352, 16), (5, 17, 33, 40, 64, 64),
+         (4, 9, 40, 47, 32, 32), (3, 10, 33, 31, 128, 128), (4, 9, 33, 31, 192, 64)]
+
+
+@pytest.mark.parametrize("shape", MARCH)
+def test_conv_march_edges(S, shape):
+    """Forward and input gradient against the oracle: 1e-5 of the max (FP32
+    sums of exact bf16 products), and operands that are only 8-byte aligned,
+    which take another kernel, within twice that."""
+    import ctypes
+    import torch
+    import _native as N
+    from oracle import conv_oracle as CO
+    nb, D, H, W, ci, co = shape
+    rng = np.random.default_rng(11 + sum(shape))
+    X = CO.bf16_round(rng.standard_normal((nb, D, H, W, ci)).astype(np.float32))
+    Wk = CO.bf16_round((0.2 * rng.standard_normal((27, co, ci))).astype(np.float32))
+    b = rng.standard_normal(co).astype(np.float32)
+    Xd, Wd, bd = _dev_bf16(X), _dev_bf16(Wk), torch.from_numpy(b).cuda()
+    Y, Yb = S.conv3d(Xd, Wd, bd, relu=True)
+    ref = np.maximum(CO.conv3d(X, Wk, b), 0)
+    assert _rel(Y.cpu().numpy(), ref) < 1e-5
+    np.testing.assert_array_equal(Yb.float().cpu().numpy(), CO.bf16_round(Y.cpu().numpy()))
+    off = torch.empty(Xd.numel() + 4, dtype=torch.bfloat16, device="cuda")
+    off[4:] = Xd.reshape(-1)
+    Yo = torch.empty_like(Y)
+    p = lambda t, o=0: ctypes.c_void_p(t.data_ptr() + o)  # noqa: E731
+    N.check(N.lib().gm_conv3d_fwd((ctypes.c_int32 * 6)(*shape), p(off, 8), p(Wd), p(bd), 1,
+                                  p(Yo), None, None))
+    torch.cuda.synchronize()
+    assert _rel(Yo.cpu().numpy(), Y.cpu().numpy()) < 2e-5
+    dY = CO.bf16_round(rng.standard_normal((nb, D, H, W, co)).astype(np.float32))
+    dX, _ = S.conv3d_bwd_data(_dev_bf16(dY), Wd, want_bf16=False)
+    torch.cuda.synchronize()
+    assert _rel(dX.cpu().numpy(), CO.conv3d_bwd_data(dY, Wk)) < 1e-5
+
+
 def test_two_layer_training_gradients(S):
     """Gradients of L = 0.5 |conv(relu(conv(X)+b1))+b2 - T|^2 through the
     kernels: with the oracle fed the same bf16-rounded intermediates, 1e-5;
