@@ -1,5 +1,5 @@
 // Types and helpers shared by the convolution kernels (gm_conv.hip,
-// gm_conv_march.hip).
+// gm_conv_march.hip, gm_conv_wgrad.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,5 +41,10 @@ bool conv_march_ok(const ConvDims& c, const void* X, const void* Wk, const void*
                    const void* Ybf);
 void launch_conv_march(const ConvDims& c, const uint16_t* X, const uint16_t* Wk,
                        const float* bias, int relu, float* Y, uint16_t* Ybf, hipStream_t s);
+
+// The weight gradient on transposing LDS reads (gm_conv_wgrad.hip).
+bool conv_wgrad_tr_ok(const ConvDims& c, const void* X, const void* dY);
+void launch_conv_wgrad_tr(const ConvDims& c, const uint16_t* X, const uint16_t* dY, float* dW,
+                          hipStream_t s);
 
 }  // namespace gm

@@ -2955,17 +2955,7 @@ extern "C" int gm_conv3d_bwd_weight(const int32_t* shape, const uint16_t* X, con
     if (!conv_shape_ok(shape)) return fail("gm_conv3d_bwd_weight: bad shape");
     if (((uintptr_t)X | (uintptr_t)dY) & 7)
         return fail("gm_conv3d_bwd_weight: X and dY must be 8-byte aligned");
-    const int64_t nvox = (int64_t)shape[0] * shape[1] * shape[2] * shape[3];
-    // about 1024 voxels per block, at most 2048 parts (grid z = 27 * parts);
-    // 4096 for 32 x 32 channels from 2^18 voxels on (each block adds its
-    // partial tile to dW with FP32 atomics: 163 us instead of 219 on 524288
-    // voxels; the other kernels were 2-6% slower with longer parts)
-    const bool long_parts = nvox >= ((int64_t)1 << 18) && shape[4] == 32 && shape[5] == 32;
-    const int64_t per = long_parts ? 4096 : 1024;
-    int64_t parts = (nvox + per - 1) / per;
-    if (parts > 2048) parts = 2048;
-    if (parts < 1) parts = 1;
-    launch_conv_wgrad(shape, X, dY, (int)parts, dW, (hipStream_t)stream);
+    launch_conv_wgrad(shape, X, dY, dW, (hipStream_t)stream);
     HIPCHK(hipGetLastError());
     return 0;
 }

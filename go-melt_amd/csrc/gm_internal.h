@@ -254,8 +254,8 @@ void launch_conv_fwd_ws(const int32_t* shape, const uint16_t* X, const uint16_t*
                         const float* bias, int relu, float* Y, uint16_t* Ybf, void* ws,
                         int64_t ws_bytes, hipStream_t s);
 void launch_conv_wflip(int ci, int co, const uint16_t* Wk, uint16_t* Wt, hipStream_t s);
-void launch_conv_wgrad(const int32_t* shape, const uint16_t* X, const uint16_t* dY, int vsplit,
-                       float* dW, hipStream_t s);
+void launch_conv_wgrad(const int32_t* shape, const uint16_t* X, const uint16_t* dY, float* dW,
+                       hipStream_t s);
 void launch_adam(float* w, uint16_t* wbf, const float* g, float* m, float* v, int64_t n, float lr,
                  float b1, float b2, float eps, int step, hipStream_t s);
 void launch_f32_to_bf16(const float* a, uint16_t* b, int64_t n, hipStream_t s);

@@ -132,6 +132,43 @@ def test_conv_march_edges(S, shape):
     assert _rel(dX.cpu().numpy(), CO.conv3d_bwd_data(dY, Wk)) < 1e-5
 
 
+# the weight gradient's edges: partial 16 x 4 and 8 x 8 columns, segments of
+# one plane and cut volumes, an odd number of columns, channel tiles off 32,
+# one voxel
+WGRAD = [(1, 1, 1, 1, 16, 16), (1, 1, 5, 17, 32, 16), (3, 2, 7, 8, 64, 48), (1, 37, 9, 15, 16, 80),
+         (2, 70, 6, 18, 32, 32), (5, 17, 33, 21, 48, 32), (3, 9, 13, 34, 96, 64)]
+
+
+@pytest.mark.parametrize("shape", WGRAD)
+def test_conv_weight_gradient_edges(S, shape):
+    """Added to what dW holds: 1e-5 of the max against the oracle (FP32 sums
+    of exact bf16 products), and operands that are only 8-byte aligned, which
+    take another kernel, within twice that."""
+    import ctypes
+    import torch
+    import _native as N
+    from oracle import conv_oracle as CO
+    nb, D, H, W, ci, co = shape
+    rng = np.random.default_rng(13 + sum(shape))
+    X = CO.bf16_round(rng.standard_normal((nb, D, H, W, ci)).astype(np.float32))
+    dY = CO.bf16_round(rng.standard_normal((nb, D, H, W, co)).astype(np.float32))
+    base = rng.standard_normal((27, co, ci)).astype(np.float32)
+    ref = CO.conv3d_bwd_weight(X, dY)
+    Xd, dYd = _dev_bf16(X), _dev_bf16(dY)
+    dW = torch.from_numpy(base.copy()).cuda()
+    S.conv3d_bwd_weight(Xd, dYd, dW)
+    off = torch.empty(Xd.numel() + 4, dtype=torch.bfloat16, device="cuda")
+    off[4:] = Xd.reshape(-1)
+    dWo = torch.zeros((27, co, ci), dtype=torch.float32, device="cuda")
+    N.check(N.lib().gm_conv3d_bwd_weight((ctypes.c_int32 * 6)(*shape),
+                                         ctypes.c_void_p(off.data_ptr() + 8),
+                                         ctypes.c_void_p(dYd.data_ptr()),
+                                         ctypes.c_void_p(dWo.data_ptr()), None))
+    torch.cuda.synchronize()
+    assert _rel(dW.cpu().numpy() - base, ref) < 1e-5
+    assert _rel(dWo.cpu().numpy(), ref) < 2e-5
+
+
 def test_two_layer_training_gradients(S):
     """Gradients of L = 0.5 |conv(relu(conv(X)+b1))+b2 - T|^2 through the
     kernels: with the oracle fed the same bf16-rounded intermediates, 1e-5;
