@@ -663,6 +663,8 @@ struct gm_engine {
     bool use_graph = true;
     bool graph_ok = false;
     hipGraphExec_t gexec = nullptr;
+    bool row_ok = false;  // the recorded single step (gm_engine_step)
+    hipGraphExec_t row_exec = nullptr;
     std::vector<void*> allocs;
 };
 
@@ -693,6 +695,7 @@ static size_t desc_bytes(int nrows) {
 extern "C" int gm_engine_destroy(gm_engine* e) {
     if (!e) return 0;
     if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
+    if (e->row_exec) (void)hipGraphExecDestroy(e->row_exec);
     for (void* p : e->allocs) (void)hipFree(p);
     for (int i = 0; i < 3; ++i)
         if (e->pair[i].blob) (void)hipFree(e->pair[i].blob);
@@ -929,13 +932,13 @@ extern "C" int gm_engine_set_layer(gm_engine* e, int64_t ne_act, int64_t nn_act,
     e->host.l1_ne_active = ne_act;
     e->host.l1_nn_active = nn_act;
     for (int i = 0; i < 4; ++i) e->host.sub[i] = sub4[i];
-    e->graph_ok = false;  // static launch arguments changed
+    e->graph_ok = e->row_ok = false;  // static launch arguments changed
     return 0;
 }
 
 extern "C" int gm_engine_use_graph(gm_engine* e, int enable) {
     e->use_graph = enable != 0;
-    e->graph_ok = false;
+    e->graph_ok = e->row_ok = false;
     return 0;
 }
 
@@ -1011,7 +1014,7 @@ extern "C" int gm_engine_load_state(gm_engine* e, const void* host, int64_t byte
         p += a.second;
     }
     // derived state: restriction path and strip layout, descriptor, tables
-    e->graph_ok = false;
+    e->graph_ok = e->row_ok = false;
     e->fast_restrict = !pairs_aligned(e);  // force update_alignment to clear partials
     if (update_alignment(e)) return -1;
     if (upload_desc(e, desc_bytes(0))) return -1;
@@ -1028,7 +1031,7 @@ extern "C" int gm_engine_set_accum_mode(gm_engine* e, int external) {
     const bool x = external != 0;
     if (x != e->acc_external) {
         e->acc_external = x;
-        e->graph_ok = false;  // the recorded step gathers/scatters Level0 or not
+        e->graph_ok = e->row_ok = false;  // the recorded step gathers/scatters Level0 or not
     }
     return 0;
 }
@@ -1055,7 +1058,7 @@ static int update_alignment(gm_engine* e) {
     const bool a = pairs_aligned(e);
     if (a != e->fast_restrict) {
         e->fast_restrict = a;
-        e->graph_ok = false;
+        e->graph_ok = e->row_ok = false;
         for (int i = 0; i < 3; ++i)
             HIPCHK(hipMemsetAsync(e->part[i], 0, pair_elems(e->pair[i].p) * 8 * sizeof(double),
                                   e->s));
@@ -1068,7 +1071,7 @@ static int update_alignment(gm_engine* e) {
         if (R0 != e->strip_R0[i] || a0 != e->strip_a0[i]) {
             e->strip_R0[i] = R0;
             e->strip_a0[i] = a0;
-            e->graph_ok = false;
+            e->graph_ok = e->row_ok = false;
         }
     }
     return 0;
@@ -1130,8 +1133,12 @@ extern "C" int gm_engine_move(gm_engine* e, const float* v, const float* vstart,
     if (update_alignment(e)) return -1;
     if (upload_desc(e, desc_bytes(0))) return -1;
     const int64_t n3 = e->nn[3], n2 = e->nn[2];
-    launch_move_l3(e->d_desc, e->T1, e->Tp2, e->Tp3, e->T3b[0], e->Tp3x, n3, e->s);
-    launch_move_l2(e->d_desc, e->T1, e->Tp2, e->T2b[0], e->Tp2x, n2, e->s);
+    {
+        MoveBufs m{e->T1,   e->Tp2,    e->Tp3,   e->T3b[0], e->Tp3x, e->T2b[0], e->Tp2x, e->L0S1,
+                   e->s2snap, e->s2box, e->S13, e->S23,    e->S12,  n3,        n2};
+        const GmPair ps[3] = {e->pair[0].p, e->pair[1].p, e->pair[2].p};
+        launch_move_all(e->d_desc, m, ps, e->s);
+    }
     {
         CopyList L;
         L.c[0] = CopyItem{e->T3, e->T3b[0], n3 * 4};
@@ -1140,12 +1147,6 @@ extern "C" int gm_engine_move(gm_engine* e, const float* v, const float* vstart,
         L.c[3] = CopyItem{e->Tp2, e->Tp2x, n2 * 4};
         launch_copy_multi(L, 4, e->s);
     }
-    {
-        const GmPair ps[3] = {e->pair[0].p, e->pair[1].p, e->pair[2].p};
-        launch_axis_tables(ps, 3, e->d_desc, e->s);
-    }
-    launch_l0_gather(e->d_desc, e->L0S1, e->s2snap, e->s2box, e->S13, e->S23, e->S12, n3, n2,
-                     e->s);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -2356,12 +2357,10 @@ static void solutions(gm_engine* e, const float* V1, const float* V2, float* T1o
     run_l3(e, e->T3, e->S13, nullptr, 0, 1.0f, T3o, 0, nullptr, nullptr);
 }
 
-extern "C" int gm_engine_step(gm_engine* e, const float* row) {
-    GmStepDesc& h = e->host;
-    h.nrows = 1;
-    for (int c = 0; c < 7; ++c) h.rows[0][c] = row[c];
-    h.dt1 = row[5];
-    if (upload_desc(e, desc_bytes(1))) return -1;
+// The single step by the general kernels: levels that are not node-aligned,
+// or a pair that the wave-brick restriction does not take.
+static void step_body_general(gm_engine* e, float dt) {
+    const GmStepDesc& h = e->host;
     GmStepDesc* d = e->d_desc;
     hipStream_t s = e->s;
     const int64_t n1 = e->nn[1], n2 = e->nn[2], n3 = e->nn[3];
@@ -2429,9 +2428,128 @@ extern "C" int gm_engine_step(gm_engine* e, const float* row) {
     hipLaunchKernelGGL(k_reset_mask, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, s,
                        e->preS2, e->S23, e->reset3, n3);
     if (!e->acc_external)
-        launch_melt_single(d, e->T3, e->preS2, e->S23, row[5], e->mat.T_liquidus, e->acc,
+        launch_melt_single(d, e->T3, e->preS2, e->S23, dt, e->mat.T_liquidus, e->acc,
                            e->macc, n3, s);
-    HIPCHK(hipGetLastError());
+}
+
+// computeSolutions (cF:2135-2204) as `solutions`, L2 and L3 with the nodal
+// properties of the step's start state (kc_of T2, T3), then the floor at T_amb.
+static void solutions_kc(gm_engine* e, const float* V1, const float* V2, float* T1o, float* T2o,
+                         float* T3o) {
+    GmStepDesc* d = e->d_desc;
+    run_l1(e, V1, T1o, GM_DT_ROW, 0.0f, 0);
+    launch_face_bc(d, 2, 1, e->cfg.level[2], T1o, T1o, e->fa2, e->fb2, e->s);
+    LSArgs a = l2_args_kc(e, e->T2, e->S12, nullptr, V2, 1.0f, T2o, 0);
+    a.clamp = 0;  // the L3 faces take the field before its floor
+    launch_row_step(a, d, e->cfg.level[2], e->d_dm, e->s);
+    launch_face_bc(d, 3, 2, e->cfg.level[3], T2o, T2o, e->fa3, e->fb3, e->s);
+    a = l3_args_kc(e, e->T3, e->S13, nullptr, 0, 1.0f, T3o, nullptr, nullptr);
+    launch_row_step(a, d, e->cfg.level[3], e->d_dm, e->s);
+    launch_clamp2(T1o, e->nn[1], T2o, e->nn[2], e->mat.T_amb, e->s);
+}
+
+// The restrictions of the three pairs of the single step as one launch's
+// items, on the carried k, cp; false when a pair is not of the form that
+// launch takes.
+static bool row_restricts(gm_engine* e, bool flux, RestrictPairs* out) {
+    RArgs r[2];  // L2, L3
+    for (int f = 2; f <= 3; ++f) {
+        if (e->nn[f] * 8 >= (int64_t)1 << 31) return false;  // 32-bit buffer offsets
+        const float *T = f == 2 ? e->T2 : e->T3, *Tp = f == 2 ? e->Tp2 : e->Tp3,
+                    *Tpx = f == 2 ? e->Tp2x : e->Tp3x;
+        const uint8_t* S1 = f == 2 ? e->S12 : e->S13;
+        r[f - 2] = flux ? rargs(e, f, T, S1, Tp, nullptr, nullptr, GM_DT_VALUE, 0, 1.0f)
+                        : rargs(e, f, T, S1, nullptr, Tpx, Tp, GM_DT_ROW, 0, 0.0f);
+    }
+    e->use_kc = true;
+    const bool ok = restrict_item(e, 1, r[1], &out->it[0]) &&
+                    restrict_item(e, 0, r[0], &out->it[1]) &&
+                    restrict_item(e, 2, r[1], &out->it[2]);
+    e->use_kc = false;
+    return ok;
+}
+
+static RowNodes row_nodes(gm_engine* e, const float* B1, float* V1, const float* B2, float* V2,
+                          bool source) {
+    const GmPair *p0 = &e->pair[0].p, *p1 = &e->pair[1].p, *p2 = &e->pair[2].p;
+    RowNodes a;
+    a.j[0] = {*p0, *p1, *p1, e->part[0], e->part[1], B1, source ? e->G1 : nullptr, V1,
+              e->gmax[1], e->w3[3]};
+    a.j[1] = {*p2, *p2, *p2, e->part[2], nullptr, B2, source ? e->G2 : nullptr, V2, e->gmax[2],
+              e->w3[3]};
+    return a;
+}
+
+// The single step on node-aligned levels.
+static void step_body_aligned(gm_engine* e, RestrictPairs& flux, RestrictPairs& mass) {
+    GmStepDesc* d = e->d_desc;
+    hipStream_t s = e->s;
+    const GmStepDesc& h = e->host;
+    const int64_t n1 = e->nn[1], n2 = e->nn[2], n3 = e->nn[3];
+    RowState st;
+    st.j[0] = {e->T3, e->S13, e->S23, e->preS2, n3, h.sub[3], kc_of(e, e->T3)};
+    st.j[1] = {e->T2, e->S12, nullptr, nullptr, n2, h.sub[2], kc_of(e, e->T2)};
+    launch_row_state(e->d_dm, st, s);
+    {
+        const GmBox& b = h.ov2;
+        const gm_grid& g3 = e->cfg.level[3];
+        RowPrep a{e->S12, e->S11,  h.sub[1],   e->pair[1].p, e->pair[2].p, e->G1,
+                  e->G2,  e->src3, e->gmax[1], e->gmax[2],   {0, 0, 0, 0}};
+        launch_row_prep(a, (int64_t)b.n[0] * b.n[1] * b.n[2], g3.n[0] + g3.n[1] + g3.n[2], d,
+                        e->d_dm, s);
+    }
+    // predictor: T' flux terms (computeCoarseTprimeTerm_jax cF:1477-1565)
+    launch_restrict_pairs(flux, true, s);
+    launch_row_nodes(row_nodes(e, nullptr, e->V1, nullptr, e->V2, true), s);
+    solutions_kc(e, e->V1, e->V2, e->T1p, e->T2b[0], e->T3b[0]);
+    new_tprime(e, 3, e->T3b[0], e->T2b[0], e->Tp3x);
+    new_tprime(e, 2, e->T2b[0], e->T1p, e->Tp2x);
+    // mass terms (computeCoarseTprimeMassTerm_jax cF:1396-1474) and corrector
+    launch_restrict_pairs(mass, false, s);
+    float* V2m = e->Tp2x;  // the L2 T' of the predictor is no longer needed
+    launch_row_nodes(row_nodes(e, e->V1, e->V1m, e->V2, V2m, false), s);
+    solutions_kc(e, e->V1m, V2m, e->T1c, e->T2b[1], e->T3b[1]);
+    // final T' (getBothNewTprimes cF:2385-2387), then the end-of-step state
+    new_tprime(e, 3, e->T3b[1], e->T2b[1], e->Tp3);
+    new_tprime(e, 2, e->T2b[1], e->T1c, e->Tp2);
+    RowClose c{e->T3b[1], e->T3,     e->S13, e->S23,
+               e->preS2,  e->L0S1,   e->s2snap, e->reset3,
+               e->s2box,  e->acc_external ? nullptr : e->acc, e->macc, n3,
+               {e->T2, e->T1}, {e->T2b[1], e->T1c}, {n2, n1}, 0};
+    launch_row_close(c, d, e->d_dm, s);
+}
+
+extern "C" int gm_engine_step(gm_engine* e, const float* row) {
+    GmStepDesc& h = e->host;
+    h.nrows = 1;
+    for (int c = 0; c < 7; ++c) h.rows[0][c] = row[c];
+    h.dt1 = row[5];
+    if (upload_desc(e, desc_bytes(1))) return -1;
+    RestrictPairs flux, mass;
+    if (!row_restricts(e, true, &flux) || !row_restricts(e, false, &mass)) {
+        step_body_general(e, row[5]);
+        HIPCHK(hipGetLastError());
+        return 0;
+    }
+    if (!e->use_graph) {
+        step_body_aligned(e, flux, mass);
+        HIPCHK(hipGetLastError());
+        return 0;
+    }
+    if (!e->row_ok) {
+        if (e->row_exec) {
+            HIPCHK(hipGraphExecDestroy(e->row_exec));
+            e->row_exec = nullptr;
+        }
+        hipGraph_t g;
+        HIPCHK(hipStreamBeginCapture(e->s, hipStreamCaptureModeThreadLocal));
+        step_body_aligned(e, flux, mass);
+        HIPCHK(hipStreamEndCapture(e->s, &g));
+        HIPCHK(hipGraphInstantiate(&e->row_exec, g, nullptr, nullptr, 0));
+        HIPCHK(hipGraphDestroy(g));
+        e->row_ok = true;
+    }
+    HIPCHK(hipGraphLaunch(e->row_exec, e->s));
     return 0;
 }
 
@@ -2508,7 +2626,7 @@ extern "C" int gm_engine_layer_change(gm_engine* e, int kidx, float new_l1_z0, f
         if (nA > 0) launch_shift_l0(e->L0S1, e->acc, nA, nB, e->nn[0], s);
         HIPCHK(hipMemsetAsync(e->macc, 0, e->nn[0] * 4, s));
     }
-    e->graph_ok = false;
+    e->graph_ok = e->row_ok = false;
     if (update_alignment(e)) return -1;
     if (upload_desc(e, desc_bytes(0))) return -1;
     HIPCHK(hipGetLastError());

@@ -376,10 +376,17 @@ void launch_inject(const GmStepDesc* d, int fine_level, int coarse_level, const 
                    float* coarseT, int64_t n_box, hipStream_t s);
 void launch_tprime(const GmStepDesc* d, int fine_level, int coarse_level, const float* fineT,
                    const float* coarseT, float* Tp, int64_t n, hipStream_t s);
-void launch_move_l3(const GmStepDesc* d, const float* T1, const float* Tp2, const float* Tp3,
-                    float* T3n, float* Tp3n, int64_t nn3, hipStream_t s);
-void launch_move_l2(const GmStepDesc* d, const float* T1, const float* Tp2, float* T2n,
-                    float* Tp2n, int64_t nn2, hipStream_t s);
+// moveEverything on the device (fields, axis tables of the three pairs, phase
+// flags) in one launch
+struct MoveBufs {
+    const float *T1, *Tp2, *Tp3;
+    float *T3n, *Tp3n, *T2n, *Tp2n;
+    const uint8_t *L0S1, *snap;
+    const int32_t* sbox;
+    uint8_t *S13, *S23, *S12;
+    int64_t nn3, nn2;
+};
+void launch_move_all(const GmStepDesc* d, const MoveBufs& m, const GmPair* ps, hipStream_t s);
 void launch_l1_s1_from_l2(const GmStepDesc* d, const uint8_t* S1_2, float* S1_1, int64_t n_box,
                           hipStream_t s);
 void launch_fill_f32(float* p, float v, int64_t n, hipStream_t s);
@@ -387,15 +394,67 @@ void launch_fill_u8(uint8_t* p, uint8_t v, int64_t n, hipStream_t s);
 void launch_copy_f32(float* dst, const float* src, int64_t n, hipStream_t s);
 void launch_copy_u8(uint8_t* dst, const uint8_t* src, int64_t n, hipStream_t s);
 void launch_clamp(float* T, int64_t n, float Tamb, hipStream_t s);
-void launch_l0_gather(const GmStepDesc* d, const uint8_t* L0S1, const uint8_t* s2snap,
-                      const int32_t* s2box, uint8_t* S1_3, uint8_t* S2_3, uint8_t* S1_2,
-                      int64_t nn3, int64_t nn2, hipStream_t s);
 void launch_l0_scatter(const GmStepDesc* d, const uint8_t* S1_3, const uint8_t* S2_3,
                        uint8_t* L0S1, uint8_t* s2snap, int32_t* s2box, int64_t nn3,
                        hipStream_t s);
 void launch_melt_single(const GmStepDesc* d, const float* T3, const uint8_t* preS2,
                         const uint8_t* S2, float dt, float Tliq, float* accum, float* max_accum,
                         int64_t nn3, hipStream_t s);
+// kernels of the single step on node-aligned levels
+struct RestrictPairs {
+    RItem it[3];
+    int b0[3];
+};
+void launch_restrict_pairs(RestrictPairs& a, bool flux, hipStream_t s);
+struct RowState {
+    struct Job {
+        const float* T;
+        uint8_t *S1, *S2, *preS2;  // S2, preS2 nullable
+        int64_t nn, n_sub;
+        float* kc;
+    } j[2];  // L3, L2
+};
+void launch_row_state(const DevMat* m, const RowState& a, hipStream_t s);
+struct RowPrep {
+    const uint8_t* S12;
+    float* S11;
+    int64_t n_sub1;
+    GmPair p1, p2;
+    float *G1, *G2, *src3;
+    int nmax1, nmax2;
+    int b[4];
+};
+void launch_row_prep(RowPrep& a, int64_t nbox, int n3axes, const GmStepDesc* d, const DevMat* m,
+                     hipStream_t s);
+// L2 (no srcT) or L3 solve of the single step, kcin from launch_row_state
+void launch_row_step(const LSArgs& a, const GmStepDesc* d, const gm_grid& hg, const DevMat* m,
+                     hipStream_t s);
+struct RowNodes {
+    struct Job {
+        GmPair po, pi, pg;
+        double *acco, *acci;  // acci nullable
+        const float *Vbase, *G;
+        float* V;
+        int nmax;
+        float scale;
+    } j[2];  // L1, L2
+};
+void launch_row_nodes(const RowNodes& a, hipStream_t s);
+void launch_clamp2(float* T0, int64_t n0, float* T1, int64_t n1, float Tamb, hipStream_t s);
+struct RowClose {
+    const float* T3o;
+    float* T3;
+    const uint8_t *S13, *S23, *preS2;
+    uint8_t *L0S1, *snap, *reset3;
+    int32_t* sbox;
+    float *accum, *max_accum;  // null: the caller keeps the melt time
+    int64_t nn3;
+    float* dst[2];  // L2, L1
+    const float* src[2];
+    int64_t n[2];
+    int bc;
+};
+void launch_row_close(RowClose& a, const GmStepDesc* d, const DevMat* m, hipStream_t s);
 void launch_minmax(const float* T, int64_t n, float* out2, hipStream_t s);
 // melt-pool size of a level's field into dims (8 floats of device memory)
 void launch_melt_pool(const gm_grid& g, const float* T, float Tl, float* dims, hipStream_t s);

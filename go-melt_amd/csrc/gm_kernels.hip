@@ -1288,11 +1288,11 @@ void launch_copy_multi(const CopyList& L, int n, hipStream_t s) {
 
 // Separable source factors of every L3 node line for the desc rows:
 // src_axis of x (times 6 sqrt(3) eta P w3), y and z (cF:1013-1025, 2986-3010).
-__global__ void k_src3_tables(const GmStepDesc* __restrict__ d, const DevMat* __restrict__ m,
-                              int nrows, float w3, float* __restrict__ out) {
+__device__ __forceinline__ void src3_table_at(const GmStepDesc* __restrict__ d,
+                                              const DevMat* __restrict__ m, int nrows, float w3,
+                                              float* __restrict__ out, int t) {
     const gm_grid& g = d->g[3];
     const int n = g.n[0] + g.n[1] + g.n[2];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nrows * n) return;
     const int r = t / n, i = t % n;
     const float* row = d->rows[r];
@@ -1305,6 +1305,11 @@ __global__ void k_src3_tables(const GmStepDesc* __restrict__ d, const DevMat* __
         v = src_axis(g, 2, i - g.n[0] - g.n[1], row[2], m->dsq, m->dc);
     }
     out[t] = v;
+}
+
+__global__ void k_src3_tables(const GmStepDesc* __restrict__ d, const DevMat* __restrict__ m,
+                              int nrows, float w3, float* __restrict__ out) {
+    src3_table_at(d, m, nrows, w3, out, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 void launch_src3_tables(const GmStepDesc* d, const DevMat* m, int nrows, int ntot, float w3,
@@ -1443,9 +1448,8 @@ struct GmPairs3 {
     GmPair p[3];
 };
 
-__global__ void k_axis_tables(GmPairs3 ps, const GmStepDesc* __restrict__ d) {
-    const GmPair& p = ps.p[blockIdx.y];
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void axis_table_at(const GmPair& p, const GmStepDesc* __restrict__ d,
+                                              int t) {
     int ax = 0;
     while (ax < 3 && t >= p.nef[ax]) {
         t -= p.nef[ax];
@@ -1483,6 +1487,10 @@ __global__ void k_axis_tables(GmPairs3 ps, const GmStepDesc* __restrict__ d) {
     }
 }
 
+__global__ void k_axis_tables(GmPairs3 ps, const GmStepDesc* __restrict__ d) {
+    axis_table_at(ps.p[blockIdx.y], d, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
 void launch_axis_tables(const GmPair* p, int np, const GmStepDesc* d, hipStream_t s) {
     GmPairs3 ps;
     int n = 0;
@@ -1501,10 +1509,10 @@ void launch_axis_tables(const GmPair* p, int np, const GmStepDesc* d, hipStream_
 // (the x table also carries 6 sqrt(3) P eta).
 // ---------------------------------------------------------------------------
 
-__global__ void k_source_tables(GmPair p, const GmStepDesc* __restrict__ d, DevMat m, int row0,
-                                int npos, int use_rows, const float* __restrict__ rows_dev,
-                                float* __restrict__ G, int nmax) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void source_table_at(const GmPair& p, const GmStepDesc* __restrict__ d,
+                                                const DevMat& m, int row0, int npos, int use_rows,
+                                                const float* __restrict__ rows_dev,
+                                                float* __restrict__ G, int nmax, int t) {
     if (t >= npos * 3 * nmax) return;
     const int A = t % nmax, ax = (t / nmax) % 3, pos = t / (3 * nmax);
     const GmAxisTab& tb = p.ax[ax];
@@ -1533,6 +1541,13 @@ __global__ void k_source_tables(GmPair p, const GmStepDesc* __restrict__ d, DevM
         if (ax == 0) s *= m.pc6 * row[6];
     }
     G[t] = s;
+}
+
+__global__ void k_source_tables(GmPair p, const GmStepDesc* __restrict__ d, DevMat m, int row0,
+                                int npos, int use_rows, const float* __restrict__ rows_dev,
+                                float* __restrict__ G, int nmax) {
+    source_table_at(p, d, m, row0, npos, use_rows, rows_dev, G, nmax,
+                    blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 void launch_source_tables(const GmPair& p, const GmStepDesc* d, const DevMat& m, int row0,
@@ -2214,6 +2229,17 @@ __global__ void __launch_bounds__(64) k_restrict_dpp_batch(const RItem* __restri
     restrict_dpp_brick<FLUX, MASS, ZC>(x.p, x.d, x.r, x.acc, b - b0);
 }
 
+// The restrictions of one engine's three pairs in one launch (the single
+// step, where all read the same start state): item i has the blocks from
+// b0[i] on.
+template <bool FLUX, bool MASS, int ZC>
+__global__ void __launch_bounds__(64) k_restrict_dpp_pairs(RestrictPairs a) {
+    const int b = xcd_tile(blockIdx.x, gridDim.x);
+    const int lo = b >= a.b0[2] ? 2 : b >= a.b0[1] ? 1 : 0;
+    const RItem& x = a.it[lo];
+    restrict_dpp_brick<FLUX, MASS, ZC>(x.p, x.d, x.r, x.acc, b - a.b0[lo]);
+}
+
 // bricks of the node-aligned restriction of pair p with arguments r
 static int restrict_dpp_nbd(const GmPair& p, const RArgs& r, int ZC) {
     const int nx = p.nef[0] + 1, ny = p.nef[1] + 1, nz = p.nef[2] + 1;
@@ -2238,6 +2264,19 @@ void launch_restrict_batch(const RItem* it, const int* bstart, int n, int nblock
     else
         hipLaunchKernelGGL((k_restrict_dpp_batch<false, true, ZC>), dim3(nblocks), dim3(64), 0, s,
                            it, bstart, n);
+}
+
+void launch_restrict_pairs(RestrictPairs& a, bool flux, hipStream_t s) {
+    constexpr int ZC = 4;
+    int n = 0;
+    for (int i = 0; i < 3; ++i) {
+        a.b0[i] = n;
+        n += restrict_dpp_nbd(a.it[i].p, a.it[i].r, ZC);
+    }
+    if (flux)
+        hipLaunchKernelGGL((k_restrict_dpp_pairs<true, false, ZC>), dim3(n), dim3(64), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_restrict_dpp_pairs<false, true, ZC>), dim3(n), dim3(64), 0, s, a);
 }
 
 void launch_restrict_fast(const GmPair& p, const GmStepDesc* d, const DevMat* m, const RArgs& r,
@@ -2703,10 +2742,11 @@ void launch_tprime_inject(const GmStepDesc* d, int fine_level, int coarse_level,
 
 // moveEverything, L3 part (cF:2439-2444): T0 = I(L1 T0) + (I(L2 T'0) + I(L3 T'0))
 // on the moved L3 nodes, with the pre-move L2 and L3 meshes.
-__global__ void k_move_l3(const GmStepDesc* __restrict__ d, const float* __restrict__ T1, const float* __restrict__ Tp2,
-                          const float* __restrict__ Tp3, float* __restrict__ T3n,
-                          float* __restrict__ Tp3n, int64_t n) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void move_l3_at(const GmStepDesc* __restrict__ d,
+                                           const float* __restrict__ T1,
+                                           const float* __restrict__ Tp2,
+                                           const float* __restrict__ Tp3, float* __restrict__ T3n,
+                                           float* __restrict__ Tp3n, int64_t n, int64_t t) {
     if (t >= n) return;
     const gm_grid& g3 = d->g[3];
     int ix, iy, iz;
@@ -2719,16 +2759,11 @@ __global__ void k_move_l3(const GmStepDesc* __restrict__ d, const float* __restr
     Tp3n[t] = c;
 }
 
-void launch_move_l3(const GmStepDesc* d, const float* T1, const float* Tp2, const float* Tp3,
-                    float* T3n, float* Tp3n, int64_t nn3, hipStream_t s) {
-    hipLaunchKernelGGL(k_move_l3, dim3((nn3 + 255) / 256), dim3(256), 0, s, d, T1, Tp2, Tp3, T3n,
-                       Tp3n, nn3);
-}
-
 // moveEverything, L2 part (cF:2460-2464)
-__global__ void k_move_l2(const GmStepDesc* __restrict__ d, const float* __restrict__ T1, const float* __restrict__ Tp2,
-                          float* __restrict__ T2n, float* __restrict__ Tp2n, int64_t n) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void move_l2_at(const GmStepDesc* __restrict__ d,
+                                           const float* __restrict__ T1,
+                                           const float* __restrict__ Tp2, float* __restrict__ T2n,
+                                           float* __restrict__ Tp2n, int64_t n, int64_t t) {
     if (t >= n) return;
     const gm_grid& g2 = d->g[2];
     int ix, iy, iz;
@@ -2740,18 +2775,13 @@ __global__ void k_move_l2(const GmStepDesc* __restrict__ d, const float* __restr
     T2n[t] = a + tp;
 }
 
-void launch_move_l2(const GmStepDesc* d, const float* T1, const float* Tp2, float* T2n,
-                    float* Tp2n, int64_t nn2, hipStream_t s) {
-    hipLaunchKernelGGL(k_move_l2, dim3((nn2 + 255) / 256), dim3(256), 0, s, d, T1, Tp2, T2n, Tp2n,
-                       nn2);
-}
-
 // L1 S1 on the L2 overlap <- interpolated L2 S1 (cF:3273-3277)
-__global__ void k_l1_s1_from_l2(const GmStepDesc* __restrict__ d, const uint8_t* __restrict__ S12,
-                                float* __restrict__ S11) {
+// (nodes below n_skip are left alone)
+__device__ __forceinline__ void l1_s1_at(const GmStepDesc* __restrict__ d,
+                                         const uint8_t* __restrict__ S12, float* __restrict__ S11,
+                                         int64_t n_skip, int t) {
     const GmBox& b = d->ov2;
     const int n = b.n[0] * b.n[1] * b.n[2];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     int ix, iy, iz;
     dec3(t, b.n[0], b.n[1], ix, iy, iz);
@@ -2765,7 +2795,13 @@ __global__ void k_l1_s1_from_l2(const GmStepDesc* __restrict__ d, const uint8_t*
     const gm_grid& g1 = d->g[1];
     const int cx = b.lo[0] + ix, cy = b.lo[1] + iy, cz = b.lo[2] + iz;
     if (cx < 0 || cx >= g1.n[0] || cy < 0 || cy >= g1.n[1] || cz < 0 || cz >= g1.n[2]) return;
-    S11[nid(cx, cy, cz, g1.n[0], g1.n[1])] = s;
+    const int64_t i = nid(cx, cy, cz, g1.n[0], g1.n[1]);
+    if (i >= n_skip) S11[i] = s;
+}
+
+__global__ void k_l1_s1_from_l2(const GmStepDesc* __restrict__ d, const uint8_t* __restrict__ S12,
+                                float* __restrict__ S11) {
+    l1_s1_at(d, S12, S11, 0, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 void launch_l1_s1_from_l2(const GmStepDesc* d, const uint8_t* S1_2, float* S1_1, int64_t n_box,
@@ -2821,11 +2857,11 @@ void launch_clamp(float* T, int64_t n, float Tamb, hipStream_t s) {
 // Level0 S2 is kept as a snapshot of the last L3 S2 and the Level0 box it was
 // written to: the reference clears all of Level0 S2 before each write, so
 // every Level0 node outside that box reads False.
-__global__ void k_l0_gather(const GmStepDesc* __restrict__ d, const uint8_t* __restrict__ L0S1,
+__device__ __forceinline__ void l0_gather_at(const GmStepDesc* __restrict__ d, const uint8_t* __restrict__ L0S1,
                             const uint8_t* __restrict__ snap, const int32_t* __restrict__ sbox,
                             uint8_t* __restrict__ S13, uint8_t* __restrict__ S23,
-                            uint8_t* __restrict__ S12, int64_t nn3, int64_t nn2) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                            uint8_t* __restrict__ S12, int64_t nn3, int64_t nn2,
+                                            int64_t t) {
     if (t < nn3) {
         const gm_grid& g3 = d->g[3];
         int ix, iy, iz;
@@ -2854,12 +2890,66 @@ __global__ void k_l0_gather(const GmStepDesc* __restrict__ d, const uint8_t* __r
     }
 }
 
-void launch_l0_gather(const GmStepDesc* d, const uint8_t* L0S1, const uint8_t* s2snap,
-                      const int32_t* s2box, uint8_t* S1_3, uint8_t* S2_3, uint8_t* S1_2,
-                      int64_t nn3, int64_t nn2, hipStream_t s) {
-    const int64_t n = nn3 > nn2 ? nn3 : nn2;
-    hipLaunchKernelGGL(k_l0_gather, dim3(nblk(n)), dim3(256), 0, s, d, L0S1, s2snap, s2box, S1_3,
-                       S2_3, S1_2, nn3, nn2);
+// moveEverything on the device, one launch: blocks below b[0] move L3, below
+// b[1] L2, below b[2] fill the pairs' axis tables, the rest gather the phase
+// flags from Level0.  All read the pre-move fields and the descriptor only.
+// Bounded by launches on small decks: 5.0 us on 41 x 41 x 21-node levels
+// (four launches of some 5 us each before), 17 us on the part-scale deck.
+struct MoveArgs {
+    const float *T1, *Tp2, *Tp3;
+    float *T3n, *Tp3n, *T2n, *Tp2n;
+    GmPairs3 ps;
+    const uint8_t *L0S1, *snap;
+    const int32_t* sbox;
+    uint8_t *S13, *S23, *S12;
+    int64_t nn3, nn2;
+    int b[3], axb;  // first block of each part; axis blocks per pair
+};
+
+__global__ void __launch_bounds__(256) k_move_all(MoveArgs a, const GmStepDesc* __restrict__ d) {
+    const int b = (int)blockIdx.x;
+    const int64_t t = threadIdx.x;
+    if (b < a.b[0]) {
+        move_l3_at(d, a.T1, a.Tp2, a.Tp3, a.T3n, a.Tp3n, a.nn3, (int64_t)b * 256 + t);
+    } else if (b < a.b[1]) {
+        move_l2_at(d, a.T1, a.Tp2, a.T2n, a.Tp2n, a.nn2, (int64_t)(b - a.b[0]) * 256 + t);
+    } else if (b < a.b[2]) {
+        const int k = b - a.b[1], pr = k / a.axb;
+        axis_table_at(a.ps.p[pr], d, (k - pr * a.axb) * 256 + (int)t);
+    } else {
+        l0_gather_at(d, a.L0S1, a.snap, a.sbox, a.S13, a.S23, a.S12, a.nn3, a.nn2,
+                     (int64_t)(b - a.b[2]) * 256 + t);
+    }
+}
+
+void launch_move_all(const GmStepDesc* d, const MoveBufs& m, const GmPair* ps, hipStream_t s) {
+    MoveArgs a;
+    a.T1 = m.T1;
+    a.Tp2 = m.Tp2;
+    a.Tp3 = m.Tp3;
+    a.T3n = m.T3n;
+    a.Tp3n = m.Tp3n;
+    a.T2n = m.T2n;
+    a.Tp2n = m.Tp2n;
+    a.L0S1 = m.L0S1;
+    a.snap = m.snap;
+    a.sbox = m.sbox;
+    a.S13 = m.S13;
+    a.S23 = m.S23;
+    a.S12 = m.S12;
+    a.nn3 = m.nn3;
+    a.nn2 = m.nn2;
+    int n = 0;
+    for (int i = 0; i < 3; ++i) {
+        a.ps.p[i] = ps[i];
+        n = std::max(n, ps[i].nef[0] + ps[i].nef[1] + ps[i].nef[2]);
+    }
+    a.axb = (n + 255) / 256;
+    a.b[0] = (int)nblk(m.nn3);
+    a.b[1] = a.b[0] + (int)nblk(m.nn2);
+    a.b[2] = a.b[1] + 3 * a.axb;
+    hipLaunchKernelGGL(k_move_all, dim3(a.b[2] + nblk(std::max(m.nn3, m.nn2))), dim3(256), 0, s,
+                       a, d);
 }
 
 __global__ void k_l0_scatter(const GmStepDesc* __restrict__ d, const uint8_t* __restrict__ S13,
@@ -2917,6 +3007,415 @@ void launch_melt_single(const GmStepDesc* d, const float* T3, const uint8_t* pre
                         int64_t nn3, hipStream_t s) {
     hipLaunchKernelGGL(k_melt_single, dim3(nblk(nn3)), dim3(256), 0, s, d, T3, preS2, S2, dt, Tliq,
                        accum, max_accum, nn3);
+}
+
+// ---------------------------------------------------------------------------
+// Kernels of the single step (stepGOMELT, cF:2304-2397) on node-aligned levels.
+// A step is a chain of small kernels, bound by their launches: independent
+// ones share a launch (block ranges), and the whole step is replayed as a
+// graph.  A row with its move took 274 us in 54 launches on 41 x 41 x 21-node
+// levels and 379 us on the part-scale deck (2.06 M L1 nodes), and takes 133
+// and 230 us in 25 recorded ones.
+// ---------------------------------------------------------------------------
+
+// updateStateProperties (cF:2513-2564) of L3 (y = 0: S1, S2, and S2 before
+// the step into preS2) and L2 (y = 1: S1), with the nodal k, cp the solves and
+// restrictions of the step read.
+__global__ void k_row_state(const DevMat* __restrict__ m, RowState a) {
+    __shared__ float sTab[PTW] __attribute__((aligned(16)));
+    stage_tables(m, sTab, threadIdx.x, blockDim.x);
+    __syncthreads();
+    const RowState::Job& J = a.j[blockIdx.y];
+    const PropC pc = load_pc(m);
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < J.nn;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const float v = J.T[i];
+        const bool s2 = v >= pc.Tliq;
+        const bool s1 = J.S1[i] != 0 || s2 || i < J.n_sub;
+        J.S1[i] = (uint8_t)s1;
+        if (J.S2) {
+            J.preS2[i] = J.S2[i];
+            J.S2[i] = (uint8_t)s2;
+        }
+        float kk, cc;
+        bool so;
+        props_c(pc, sTab, v, s1, false, kk, cc, so);
+        J.kc[i] = kk;
+        J.kc[J.nn + i] = cc;
+    }
+}
+
+void launch_row_state(const DevMat* m, const RowState& a, hipStream_t s) {
+    const int64_t nb = std::min<int64_t>((std::max(a.j[0].nn, a.j[1].nn) + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_row_state, dim3((unsigned)nb, 2), dim3(256), 0, s, m, a);
+}
+
+// L1 S1 from the new L2 S1 and the substrate (cF:3273-3278), the row's source
+// tables onto L1 and L2 and its L3 source factors, in block ranges.
+__global__ void __launch_bounds__(256) k_row_prep(RowPrep a, const GmStepDesc* __restrict__ d,
+                                                  const DevMat* __restrict__ m) {
+    const int b = (int)blockIdx.x, t = (int)threadIdx.x;
+    if (b < a.b[0]) {
+        l1_s1_at(d, a.S12, a.S11, a.n_sub1, b * 256 + t);
+    } else if (b < a.b[1]) {
+        const int64_t i = (int64_t)(b - a.b[0]) * 256 + t;
+        if (i < a.n_sub1) a.S11[i] = 1.0f;
+    } else if (b < a.b[2]) {
+        source_table_at(a.p1, d, *m, 0, 1, 0, nullptr, a.G1, a.nmax1, (b - a.b[1]) * 256 + t);
+    } else if (b < a.b[3]) {
+        source_table_at(a.p2, d, *m, 0, 1, 0, nullptr, a.G2, a.nmax2, (b - a.b[2]) * 256 + t);
+    } else {
+        src3_table_at(d, m, 1, 1.0f, a.src3, (b - a.b[3]) * 256 + t);
+    }
+}
+
+void launch_row_prep(RowPrep& a, int64_t nbox, int n3axes, const GmStepDesc* d, const DevMat* m,
+                     hipStream_t s) {
+    a.b[0] = (int)nblk(nbox);
+    a.b[1] = a.b[0] + (int)nblk(a.n_sub1);
+    a.b[2] = a.b[1] + (int)nblk(3 * a.nmax1);
+    a.b[3] = a.b[2] + (int)nblk(3 * a.nmax2);
+    hipLaunchKernelGGL(k_row_prep, dim3(a.b[3] + nblk(n3axes)), dim3(256), 0, s, a, d, m);
+}
+
+// The corrections of L1 (y = 0: outer box L2 -> L1, inner box L3 -> L1) and L2
+// (y = 1): k_restrict_nodes_acc's sum, the source of the step's one laser
+// position taken from its tables.  The boxes are cleared as they are read;
+// threads past the outer box clear the inner nodes that no outer node reads.
+__global__ void k_row_nodes(RowNodes a) {
+    const RowNodes::Job& J = a.j[blockIdx.y];
+    const GmPair &po = J.po, &pi = J.pi, &pg = J.pg;
+    const int mx = po.cmax[0] + 1, my = po.cmax[1] + 1, mz = po.cmax[2] + 1;
+    const int no = mx * my * mz;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int ix1 = pi.cmax[0] + 1, iy1 = pi.cmax[1] + 1, iz1 = pi.cmax[2] + 1;
+    if (t >= no) {
+        const int u = t - no;
+        if (!J.acci || u >= ix1 * iy1 * iz1) return;
+        const int B[3] = {u % ix1, (u / ix1) % iy1, u / (ix1 * iy1)};
+        bool read = true;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int o = pi.ax[k].info[0] + B[k] - po.ax[k].info[0];
+            read = read && B[k] <= pi.ax[k].info[1] && o >= 0 && o <= po.cmax[k];
+        }
+        if (!read) J.acci[u] = 0.0;
+        return;
+    }
+    const int bx = t % mx, by = (t / mx) % my, bz = t / (mx * my);
+    const int A[3] = {po.ax[0].info[0] + bx, po.ax[1].info[0] + by, po.ax[2].info[0] + bz};
+    double s = J.acco[t];
+    J.acco[t] = 0.0;
+    if (J.acci) {
+        const int ix = A[0] - pi.ax[0].info[0], iy = A[1] - pi.ax[1].info[0],
+                  iz = A[2] - pi.ax[2].info[0];
+        if (ix >= 0 && ix <= pi.ax[0].info[1] && iy >= 0 && iy <= pi.ax[1].info[1] && iz >= 0 &&
+            iz <= pi.ax[2].info[1]) {
+            const int k = ix + ix1 * (iy + iy1 * iz);
+            s += J.acci[k];
+            J.acci[k] = 0.0;
+        }
+    }
+    float v = (J.Vbase ? J.Vbase[t] : 0.0f) + (float)s;
+    if (J.G) {
+        const int gx = A[0] - pg.ax[0].info[0], gy = A[1] - pg.ax[1].info[0],
+                  gz = A[2] - pg.ax[2].info[0];
+        if (gx >= 0 && gx <= pg.ax[0].info[1] && gy >= 0 && gy <= pg.ax[1].info[1] && gz >= 0 &&
+            gz <= pg.ax[2].info[1])
+            v += (J.G[gx] * J.G[J.nmax + gy] * J.G[2 * J.nmax + gz]) * J.scale;
+    }
+    J.V[t] = v;
+}
+
+void launch_row_nodes(const RowNodes& a, hipStream_t s) {
+    int n = 1;
+    for (int i = 0; i < 2; ++i) {
+        const auto box = [](const GmPair& p) {
+            return (p.cmax[0] + 1) * (p.cmax[1] + 1) * (p.cmax[2] + 1);
+        };
+        n = std::max(n, box(a.j[i].po) + (a.j[i].acci ? box(a.j[i].pi) : 0));
+    }
+    hipLaunchKernelGGL(k_row_nodes, dim3((n + 255) / 256, 2), dim3(256), 0, s, a);
+}
+
+// Floor at T_amb of two fields (y picks one), 16 bytes at a time.
+__global__ void k_clamp2(float* T0, int64_t n0, float* T1, int64_t n1, float Tamb) {
+    float* T = blockIdx.y ? T1 : T0;
+    const int64_t n = blockIdx.y ? n1 : n0;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (i + 3 < n) {
+        float4 v = *(const float4*)(T + i);
+        if (v.x < Tamb || v.y < Tamb || v.z < Tamb || v.w < Tamb) {
+            if (v.x < Tamb) v.x = Tamb;
+            if (v.y < Tamb) v.y = Tamb;
+            if (v.z < Tamb) v.z = Tamb;
+            if (v.w < Tamb) v.w = Tamb;
+            *(float4*)(T + i) = v;
+        }
+    } else {
+        for (int64_t k = i; k < n; ++k)
+            if (T[k] < Tamb) T[k] = Tamb;
+    }
+}
+
+void launch_clamp2(float* T0, int64_t n0, float* T1, int64_t n1, float Tamb, hipStream_t s) {
+    hipLaunchKernelGGL(k_clamp2, dim3(nblk((std::max(n0, n1) + 3) / 4), 2), dim3(256), 0, s, T0,
+                       n0, T1, n1, Tamb);
+}
+
+// a * b rounded by itself, never fused into a sum that reads it
+__device__ __forceinline__ float mul_rounded(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
+// Fine-level (L2, L3) solve of the single step on the nodal k, cp of
+// k_row_state: k_step_dpp's wave layout and neighbour access, with the sums
+// and the update in k_level_step's order (k_step_dpp's own form rounds the
+// update differently; over 40 rows the part deck's L2 T' then drifts 3e-5 from
+// the general path, with this form 5e-6).
+template <bool SRC, int ZC>
+__global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __restrict__ d,
+                                                 const DevMat* __restrict__ m) {
+    const int nx = a.grid.n[0], ny = a.grid.n[1], nz = a.grid.n[2];
+    const int nxy = nx * ny, nn = nxy * nz;
+    const int nex = nx - 1, ney = ny - 1, nez = nz - 1;
+    const int nzc = (nz + ZC - 1) / ZC;
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int qs = t / nzc, z0 = (t - qs * nzc) * ZC;
+    const int lane = (int)threadIdx.x;
+    const int q = DXS * qs - 1 + lane;
+    const bool qv = q >= 0 && q < nxy;
+    const int y = qv ? (int)((unsigned)q / (unsigned)nx) : 0;
+    const int x = qv ? q - y * nx : -1;
+    const bool ein = qv && x < nex;
+    const bool olane = lane >= 1 && lane <= DXS && qv;
+    const int base = x + nx * y + nxy * z0;
+    const uint32_t nb4 = (uint32_t)nn * 4u;
+
+    // ---- loads: planes z0-1 .. z0+ZC, rows y-1 .. y+1 ------------------------
+    const auto rT = buf_rsrc(a.T, nb4), rKC = buf_rsrc(a.kcin, 2u * nb4);
+    const auto rFa = buf_rsrc(a.bcA, nb4), rFb = buf_rsrc(a.bcB, nb4);
+    float Tw[ZC + 2][3], Kw[ZC + 2][3], Cw[ZC + 2][3];
+#pragma unroll
+    for (int p = 0; p < ZC + 2; ++p) {
+        const int zz = z0 - 1 + p;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int yy = y - 1 + r;
+            const bool ok = qv && yy >= 0 && yy < ny && zz >= 0 && zz < nz;
+            const uint32_t vo =
+                ok ? 4u * (uint32_t)(base + nx * (r - 1) + nxy * (p - 1)) : GM_OOB;
+            Tw[p][r] = buf_ld(rT, vo);
+            Kw[p][r] = buf_ld(rKC, vo);
+            Cw[p][r] = buf_ld(rKC, vo, nb4);
+        }
+    }
+    float corr[ZC], fa[ZC], fb[ZC];
+    uint32_t oF[ZC];
+    bool face[ZC];
+#pragma unroll
+    for (int i = 0; i < ZC; ++i) {
+        const int zz = z0 + i;
+        const bool ok = olane && zz < nz;
+        face[i] = x == 0 || x == nex || y == 0 || y == ney || zz == 0;
+        oF[i] = ok ? 4u * (uint32_t)(base + nxy * i) : GM_OOB;
+        const uint32_t fo = face[i] ? oF[i] : GM_OOB;
+        fa[i] = buf_ld(rFa, fo);
+        fb[i] = buf_ld(rFb, fo);
+        corr[i] = 0.0f;
+        if (!SRC) {
+            const int bx = x - a.corr_info[0][0], by = y - a.corr_info[1][0],
+                      bz = zz - a.corr_info[2][0];
+            if (ok && bx >= 0 && bx <= a.corr_info[0][1] && by >= 0 && by <= a.corr_info[1][1] &&
+                bz >= 0 && bz <= a.corr_info[2][1])
+                corr[i] = a.corr[bx + a.corr_nmax[0] * (by + a.corr_nmax[1] * bz)];
+        }
+    }
+    float sx = 0.0f, sy = 0.0f, sz[ZC];
+    if (SRC) {
+        sx = qv ? a.srcT[x] : 0.0f;
+        sy = qv ? a.srcT[nx + y] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < ZC; ++i) sz[i] = z0 + i < nz ? a.srcT[nx + ny + z0 + i] : 0.0f;
+    }
+    const float mfac = a.mrow / d->rows[0][5];
+    const float Tamb = m->T_amb;
+
+    // ---- element means: x pairs, then y, then z -------------------------------
+    float Ek[ZC + 1][2], Ec[ZC + 1][2];
+    {
+        float Sk[ZC + 2][2], Sc[ZC + 2][2];
+#pragma unroll
+        for (int p = 0; p < ZC + 2; ++p) {
+            float hk[3], hc[3];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                hk[r] = Kw[p][r] + lane_next(Kw[p][r]);
+                hc[r] = Cw[p][r] + lane_next(Cw[p][r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                Sk[p][r] = hk[r] + hk[r + 1];
+                Sc[p][r] = hc[r] + hc[r + 1];
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < ZC + 1; ++p) {
+            const int ez = z0 - 1 + p;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int ey = y - 1 + r;
+                const bool ok = ein && ey >= 0 && ey < ney && ez >= 0 && ez < nez;
+                Ek[p][r] = ok ? (Sk[p][r] + Sk[p + 1][r]) * 0.125f : 0.0f;
+                Ec[p][r] = ok ? (Sc[p][r] + Sc[p + 1][r]) * 0.125f : 0.0f;
+            }
+        }
+    }
+    // ---- surface flux of the nodes of the top plane (cF:2207-2301) ------------
+    float Ftop = 0.0f;
+    const int ptop = nez - (z0 - 1);  // window plane of the top plane
+    if (ptop >= 1 && ptop <= ZC) {
+        float Fq[2][4];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            float t0 = 0.0f, t3 = 0.0f;
+#pragma unroll
+            for (int p = 1; p <= ZC; ++p)
+                if (p == ptop) {
+                    t0 = Tw[p][r];
+                    t3 = Tw[p][r + 1];
+                }
+            const float t1 = lane_next(t0), t2 = lane_next(t3);
+            const int ey = y - 1 + r;
+            const bool ok = ein && ey >= 0 && ey < ney;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float Tq = n2(g, 0) * t0 + n2(g, 1) * t1 + n2(g, 2) * t2 + n2(g, 3) * t3;
+                Fq[r][g] = ok ? face_flux(*m, Tq) * a.w2 : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int bx = e & 1, by = e >> 1;  // 0: face on the negative side
+            const int ai = by ? (bx ? 0 : 1) : (bx ? 3 : 2);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float v = Fq[by][g];
+                Ftop += n2(g, ai) * (bx ? v : lane_prev(v));
+            }
+        }
+    }
+
+    const auto rTo = buf_rsrc(a.Tout, nb4);
+#pragma unroll
+    for (int i = 0; i < ZC; ++i) {
+        const float k100 = Ek[i][0], k110 = Ek[i][1];
+        const float k101 = Ek[i + 1][0], k111 = Ek[i + 1][1];
+        const float k000 = lane_prev(k100), k010 = lane_prev(k110);
+        const float k001 = lane_prev(k101), k011 = lane_prev(k111);
+        const float Msum = ((lane_prev(Ec[i][0]) + Ec[i][0]) + (lane_prev(Ec[i][1]) + Ec[i][1])) +
+                           ((lane_prev(Ec[i + 1][0]) + Ec[i + 1][0]) +
+                            (lane_prev(Ec[i + 1][1]) + Ec[i + 1][1]));
+        const float Pz00 = k000 + k001, Pz10 = k100 + k101, Pz01 = k010 + k011, Pz11 = k110 + k111;
+        const float Py00 = k000 + k010, Py10 = k100 + k110, Py01 = k001 + k011, Py11 = k101 + k111;
+        const float Px00 = k000 + k100, Px10 = k010 + k110, Px01 = k001 + k101, Px11 = k011 + k111;
+        const float Fx0 = Pz00 + Pz01, Fx1 = Pz10 + Pz11;
+        const float Fy0 = Pz00 + Pz10, Fy1 = Pz01 + Pz11;
+        const float Fz0 = Py00 + Py10, Fz1 = Py01 + Py11;
+        const float Kc = Fx0 + Fx1;
+        const float Ti = Tw[i + 1][1];
+        const auto P = [&](int p, int r) { return lane_prev(Tw[p][r]); };
+        const auto N = [&](int p, int r) { return lane_next(Tw[p][r]); };
+        float KT = a.kc[0] * (Kc * Ti);
+        KT += a.kc[1] * (Fx0 * P(i + 1, 1) + Fx1 * N(i + 1, 1));
+        KT += a.kc[2] * (Fy0 * Tw[i + 1][0] + Fy1 * Tw[i + 1][2]);
+        KT += a.kc[4] * (Fz0 * Tw[i][1] + Fz1 * Tw[i + 2][1]);
+        KT += a.kc[3] * (Pz00 * P(i + 1, 0) + Pz10 * N(i + 1, 0) + Pz01 * P(i + 1, 2) +
+                         Pz11 * N(i + 1, 2));
+        KT += a.kc[5] * (Py00 * P(i, 1) + Py10 * N(i, 1) + Py01 * P(i + 2, 1) + Py11 * N(i + 2, 1));
+        KT += a.kc[6] * (Px00 * Tw[i][0] + Px10 * Tw[i][2] + Px01 * Tw[i + 2][0] +
+                         Px11 * Tw[i + 2][2]);
+        KT += a.kc[7] * (k000 * P(i, 0) + k100 * N(i, 0) + k010 * P(i, 2) + k110 * N(i, 2) +
+                         k001 * P(i + 2, 0) + k101 * N(i + 2, 0) + k011 * P(i + 2, 2) +
+                         k111 * N(i + 2, 2));
+        const float M = Msum * mfac;
+        float F = 0.0f;
+        if (SRC) F = mul_rounded(sx * sy * sz[i], a.w3);
+        if (i + 1 == ptop) F += Ftop;
+        float Tnew = ((M * Ti - KT) + F + corr[i]) / M;
+        if (face[i]) Tnew = a.alpha * fa[i] + (1.0f - a.alpha) * fb[i];
+        if (a.clamp && Tnew < Tamb) Tnew = Tamb;
+        buf_st(Tnew, rTo, oF[i]);
+    }
+}
+
+void launch_row_step(const LSArgs& a0, const GmStepDesc* d, const gm_grid& hg, const DevMat* m,
+                     hipStream_t s) {
+    LSArgs a = a0;
+    a.grid = hg;
+    // planes per wave as launch_dpp
+    if (a.srcT)
+        hipLaunchKernelGGL((k_row_step<true, 3>), dim3(batch_bricks(hg, 1, 3)), dim3(64), 0, s, a,
+                           d, m);
+    else
+        hipLaunchKernelGGL((k_row_step<false, 2>), dim3(batch_bricks(hg, 1, 2)), dim3(64), 0, s, a,
+                           d, m);
+}
+
+// End of the single step, per L3 node: the new T0, Level0 S1 and the S2
+// snapshot (cF:2390-2392), the reset mask (cF:2394-2397) and, unless the
+// caller keeps them, the melt-time maps (go_melt.py:339-357).  Blocks from bc
+// on copy the new L2 and L1 fields.
+__global__ void __launch_bounds__(256) k_row_close(RowClose a, const GmStepDesc* __restrict__ d,
+                                                   const DevMat* __restrict__ m) {
+    if ((int)blockIdx.x >= a.bc) {
+        const int64_t i = (int64_t)((int)blockIdx.x - a.bc) * 256 + threadIdx.x;
+        for (int k = 0; k < 2; ++k) {
+            const int64_t n4 = a.n[k] >> 2;
+            if (i < n4) ((float4*)a.dst[k])[i] = ((const float4*)a.src[k])[i];
+            if (i < a.n[k] - 4 * n4) a.dst[k][4 * n4 + i] = a.src[k][4 * n4 + i];
+        }
+        return;
+    }
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= a.nn3) return;
+    const gm_grid& g3 = d->g[3];
+    int ix, iy, iz;
+    dec3(t, g3.n[0], g3.n[1], ix, iy, iz);
+    const int lx = d->l0_lo3[0] + ix, ly = d->l0_lo3[1] + iy, lz = d->l0_lo3[2] + iz;
+    const bool in0 = lx >= 0 && lx < d->l0_n[0] && ly >= 0 && ly < d->l0_n[1] && lz >= 0 &&
+                     lz < d->l0_n[2];
+    const int64_t l0 = in0 ? nid(lx, ly, lz, d->l0_n[0], d->l0_n[1]) : 0;
+    const float T = a.T3o[t];
+    const uint8_t s2 = a.S23[t];
+    const bool reset = a.preS2[t] == 0 && s2 != 0;
+    a.T3[t] = T;
+    a.snap[t] = s2;
+    a.reset3[t] = (uint8_t)reset;
+    if (in0) {
+        a.L0S1[l0] = a.S13[t];
+        if (a.accum) {
+            float acc = a.accum[l0];
+            const float racc = reset ? acc : 0.0f;
+            const float mx = a.max_accum[l0];
+            a.max_accum[l0] = racc > mx ? racc : mx;
+            acc = acc - racc;
+            a.accum[l0] = acc + ((T > m->T_liq) ? 1.0f : 0.0f) * d->rows[0][5];
+        }
+    }
+    if (t == 0) {
+        a.sbox[0] = d->l0_lo3[0];
+        a.sbox[1] = d->l0_lo3[1];
+        a.sbox[2] = d->l0_lo3[2];
+        a.sbox[3] = 1;
+    }
+}
+
+void launch_row_close(RowClose& a, const GmStepDesc* d, const DevMat* m, hipStream_t s) {
+    a.bc = (int)nblk(a.nn3);
+    hipLaunchKernelGGL(k_row_close, dim3(a.bc + nblk((std::max(a.n[0], a.n[1]) + 3) / 4)),
+                       dim3(256), 0, s, a, d, m);
 }
 
 // min / max with NaN propagation (printLevelMaxMin, cF:3635-3665)

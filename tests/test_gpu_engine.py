@@ -122,6 +122,24 @@ def test_driver_vs_oracle(oracle, tmp_path, case):
         assert abs(pg[0] - po[0]) <= 0.05 * float(h[2]), (pg, po)
 
 
+# planes smaller than one 62-lane strip, a strip and a remainder, rows of 61
+# nodes; 3, 5, 7 planes against bricks of 2 and 3
+@pytest.mark.parametrize("n,dt3,track", [((4, 4, 2), 1e-3, 1.5), ((8, 12, 4), 5e-4, 0.6),
+                                         ((16, 8, 6), 2e-4, 0.3), ((60, 4, 2), 1e-5, 0.03)])
+def test_single_steps_vs_oracle(oracle, tmp_path, n, dt3, track):
+    """A toolpath of single steps only (shorter than one subcycled chunk);
+    bounds as the driver test above."""
+    inp, g = W.tiny(n=n, n2=5, n3=8, track=track, dt3=dt3,
+                    props={"laser_power": 600.0, "emissivity": 0.4,
+                           "thermal_conductivity_bulk_table": W.K_TABLE,
+                           "heat_capacity_solid_table": W.CP_TABLE})
+    out, st = _run_both(oracle, inp, g, tmp_path)
+    assert st["subcycle"] == 0 and st["single"] >= 10
+    for k in (1, 2, 3):
+        a, b = out[k]
+        assert _relT(a, b) < 5e-4, (k, _relT(a, b))
+
+
 def test_driver_vs_oracle_unaligned_windows(oracle, tmp_path):
     """L2 origin a quarter of an L1 spacing off the L1 nodes: the coarse
     overlap nodes are not fine nodes, so the engine takes the general
