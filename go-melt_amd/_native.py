@@ -152,17 +152,21 @@ _SIGS = {
     "gm_conv3d_fwd": (_I, [_IP, _P, _P, _P, _I, _P, _P, _P]),
     "gm_conv3d_fwd_ws_bytes": (_I, [_IP, C.POINTER(_I64)]),
     "gm_conv3d_fwd_ws": (_I, [_IP, _P, _P, _P, _I, _P, _P, _P, _I64, _P]),
+    "gm_conv3d_fwd_bf16": (_I, [_IP, _P, _P, _P, _I, _P, _P, _I64, _P]),
     "gm_conv3d_bwd_data": (_I, [_IP, _P, _P, _P, _P, _P, _P]),
     "gm_conv3d_bwd_weight": (_I, [_IP, _P, _P, _P, _P]),
     "gm_adam": (_I, [_P, _P, _P, _P, _P, _I64, _F, _F, _F, _F, _I, _P]),
     "gm_f32_to_bf16": (_I, [_P, _P, _I64, _P]),
     "gm_nn_pool2": (_I, [_I, _IP, _P, _P, _P]),
     "gm_nn_up2": (_I, [_I, _IP, _P, _P, _P]),
+    "gm_nn_up2_concat": (_I, [_IP, _I, _P, _P, _P, _P]),
+    "gm_nn_up2_bwd": (_I, [_IP, _I, _P, _P, _P]),
     "gm_nn_concat": (_I, [_I64, _I, _I, _P, _P, _P, _P]),
     "gm_nn_split": (_I, [_I64, _I, _I, _P, _P, _P, _P]),
     "gm_nn_relu_bwd": (_I, [_I64, _P, _P, _P, _P, _P, _P]),
     "gm_nn_bias_grad": (_I, [_I64, _I, _P, _P, _P]),
     "gm_nn_relu_bias_bwd": (_I, [_I64, _I, _P, _P, _P, _P, _P, _P, _P]),
+    "gm_nn_relu_bias_net": (_I, [_IP, _P, _I, _P, _I64, _P, _P, _P, _P]),
     "gm_nn_mse": (_I, [_I64, _I, _P, _P, _P, _P, _P]),
     "gm_nn_window_input": (_I, [_IP, _FP, _P, _P, _FP, _P, _P]),
     "gm_nn_window_apply": (_I, [_IP, _P, _P, _P, _I, _F, _F, _P, _P]),

@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(ConvDims c, const uint16_t* __
                 if (v < c.nvox && o < c.co) {
                     float y = acc[a][b][r] + (bias ? bias[o] : 0.0f);
                     if (relu && y < 0.0f) y = 0.0f;
-                    Y[v * c.co + o] = y;
+                    if (Y) Y[v * c.co + o] = y;
                     if (Ybf) Ybf[v * c.co + o] = f2bf(y);
                 }
             }
@@ -276,7 +276,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd32(ConvDims c, const uint16_t* 
                     }
                     float y = acc[a][b][r] + (bias ? bias[oo] : 0.0f);
                     if (relu && y < 0.0f) y = 0.0f;
-                    Y[v * c.co + oo] = y;
+                    if (Y) Y[v * c.co + oo] = y;
                     if (Ybf) Ybf[v * c.co + oo] = f2bf(y);
                 }
             }
@@ -292,7 +292,7 @@ __global__ void k_conv_part_sum(const float* __restrict__ part, int S, int64_t n
     for (int z = 0; z < S; ++z) y += part[(int64_t)z * n + t];
     if (bias) y += bias[t % co];
     if (relu && y < 0.0f) y = 0.0f;
-    Y[t] = y;
+    if (Y) Y[t] = y;
     if (Ybf) Ybf[t] = f2bf(y);
 }
 

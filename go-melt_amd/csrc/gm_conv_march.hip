@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(64 * WV, 2)
                     for (int r = 0; r < 4; ++r)
                         if (v[r] < 0.0f) v[r] = 0.0f;
                 }
-                *(v4f*)(Y + i) = v;
+                if (Y) *(v4f*)(Y + i) = v;
                 if (Ybf) {
                     uint2 h;
                     h.x = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);

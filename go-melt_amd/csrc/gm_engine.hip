@@ -3054,6 +3054,21 @@ extern "C" int gm_conv3d_fwd_ws(const int32_t* shape, const uint16_t* X, const u
     return 0;
 }
 
+extern "C" int gm_conv3d_fwd_bf16(const int32_t* shape, const uint16_t* X, const uint16_t* Wk,
+                                  const float* bias, int relu, uint16_t* Ybf, void* ws,
+                                  int64_t ws_bytes, void* stream) {
+    if (!shape || !X || !Wk || !Ybf) return fail("gm_conv3d_fwd_bf16: null argument");
+    if (!conv_shape_ok(shape))
+        return fail("gm_conv3d_fwd_bf16: shape {nb, D, H, W, cin, cout} needs positive sizes and "
+                    "channel counts that are multiples of 16");
+    if (((uintptr_t)X | (uintptr_t)Wk) & 7)
+        return fail("gm_conv3d_fwd_bf16: X and Wk must be 8-byte aligned (4 bf16 per load)");
+    if (ws && ((uintptr_t)ws & 15)) return fail("gm_conv3d_fwd_bf16: ws must be 16-byte aligned");
+    launch_conv_fwd_ws(shape, X, Wk, bias, relu, nullptr, Ybf, ws, ws_bytes, (hipStream_t)stream);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 extern "C" int gm_conv3d_bwd_data(const int32_t* shape, const uint16_t* dY, const uint16_t* Wk,
                                   uint16_t* Wt_work, float* dX, uint16_t* dXbf, void* stream) {
     if (!shape || !dY || !Wk || !Wt_work || !dX) return fail("gm_conv3d_bwd_data: null argument");
@@ -3119,6 +3134,26 @@ extern "C" int gm_nn_up2(int dir, const int32_t* coarse_shape, const void* in, v
     return 0;
 }
 
+extern "C" int gm_nn_up2_concat(const int32_t* coarse_shape, int ca, const uint16_t* A,
+                                const uint16_t* X, uint16_t* Y, void* stream) {
+    if (!shape5_ok(coarse_shape) || ca < 1 || !A || !X || !Y)
+        return fail("gm_nn_up2_concat: bad arguments");
+    const int32_t* c = coarse_shape;
+    launch_nn_up2_concat(c[0], c[1], c[2], c[3], ca, c[4], A, X, Y, (hipStream_t)stream);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+extern "C" int gm_nn_up2_bwd(const int32_t* coarse_shape, int ld, const float* dY, float* dX,
+                             void* stream) {
+    if (!shape5_ok(coarse_shape) || ld < coarse_shape[4] || !dY || !dX)
+        return fail("gm_nn_up2_bwd: bad arguments");
+    const int32_t* c = coarse_shape;
+    launch_nn_up2_bwd(c[0], c[1], c[2], c[3], c[4], ld, dY, dX, (hipStream_t)stream);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 extern "C" int gm_nn_concat(int64_t nvox, int ca, int cb, const uint16_t* A, const uint16_t* B,
                             uint16_t* Y, void* stream) {
     if (nvox < 0 || ca < 1 || cb < 1 || !A || !B || !Y) return fail("gm_nn_concat: bad arguments");
@@ -3160,6 +3195,27 @@ extern "C" int gm_nn_relu_bias_bwd(int64_t nvox, int C, const float* dA, const f
         if ((uintptr_t)ptrs[i] & (i == 4 ? 7 : 15))
             return fail("gm_nn_relu_bias_bwd: operands must be 16-byte (dZb 8-byte) aligned");
     if (nvox) launch_nn_relu_bias_bwd(nvox, C, dA, dA2, A, dZ, dZb, db, (hipStream_t)stream);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+extern "C" int gm_nn_relu_bias_net(const int32_t* shape, const float* dA, int pooled,
+                                   const float* dA2, int64_t ld2, const uint16_t* A,
+                                   uint16_t* dZb, float* db, void* stream) {
+    if (!shape5_ok(shape) || !dA || !A || !dZb || !db)
+        return fail("gm_nn_relu_bias_net: bad arguments");
+    const int C = shape[4];
+    if (C < 4 || C > 256 || (C & 3) || 256 % C)
+        return fail("gm_nn_relu_bias_net: C must be a multiple of 4 that divides 256");
+    if ((int64_t)shape[0] * shape[1] * shape[2] * shape[3] >= (int64_t)1 << 31)
+        return fail("gm_nn_relu_bias_net: more than 2^31 - 1 voxels");
+    if (pooled && ((shape[1] | shape[2] | shape[3]) & 1))
+        return fail("gm_nn_relu_bias_net: a pooled gradient needs even extents");
+    if (dA2 && (ld2 < C || (ld2 & 3)))
+        return fail("gm_nn_relu_bias_net: ld2 must be a multiple of 4, at least C");
+    if ((((uintptr_t)dA | (uintptr_t)dA2) & 15) || (((uintptr_t)A | (uintptr_t)dZb) & 7))
+        return fail("gm_nn_relu_bias_net: FP32 operands must be 16-byte, bf16 8-byte aligned");
+    launch_nn_relu_bias_net(shape, dA, pooled, dA2, ld2, A, dZb, db, (hipStream_t)stream);
     HIPCHK(hipGetLastError());
     return 0;
 }

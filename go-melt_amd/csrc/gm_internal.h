@@ -272,6 +272,13 @@ void launch_nn_split(int64_t nvox, int ca, int cb, const float* dY, float* dA, f
 void launch_nn_relu_bwd(int64_t n, const float* dA, const float* dA2, const float* A, float* dZ,
                         uint16_t* dZb, hipStream_t s);
 void launch_nn_bias_grad(int64_t nvox, int C, const float* dZ, float* db, hipStream_t s);
+void launch_nn_up2_bwd(int nb, int D, int H, int W, int C, int ld, const float* dY, float* dX,
+                       hipStream_t s);
+void launch_nn_up2_concat(int nb, int D, int H, int W, int ca, int cb, const uint16_t* A,
+                          const uint16_t* X, uint16_t* Y, hipStream_t s);
+void launch_nn_relu_bias_net(const int32_t* shape, const float* dA, int pooled, const float* dA2,
+                             int64_t ld2, const uint16_t* A, uint16_t* dZb, float* db,
+                             hipStream_t s);
 void launch_nn_relu_bias_bwd(int64_t nvox, int C, const float* dA, const float* dA2,
                              const float* A, float* dZ, uint16_t* dZb, float* db, hipStream_t s);
 void launch_nn_mse(int64_t nvox, int C, const float* Y, const float* target, float* dY,

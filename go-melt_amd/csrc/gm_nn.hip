@@ -94,8 +94,20 @@ __global__ void k_up2(int nb, int D, int H, int W, int C, const V* __restrict__ 
     Y[t] = X[((((int64_t)b * D + z / 2) * H + y / 2) * W + x / 2) * C + c];
 }
 
-__global__ void k_up2_bwd(int nb, int D, int H, int W, int C, const float* __restrict__ dY,
-                          float* __restrict__ dX) {
+__device__ __forceinline__ void nn_add(float& a, float b) { a += b; }
+__device__ __forceinline__ void nn_add(float4& a, float4 b) {
+    a.x += b.x;
+    a.y += b.y;
+    a.z += b.z;
+    a.w += b.w;
+}
+
+// V is float, or float4 with C and ld (elements from one voxel of dY to the
+// next: more than C for the upper channels of a wider gradient) in groups of
+// four channels
+template <typename V>
+__global__ void k_up2_bwd(int nb, int D, int H, int W, int C, int ld, const V* __restrict__ dY,
+                          V* __restrict__ dX) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t n = (int64_t)nb * D * H * W * C;
     if (t >= n) return;
@@ -108,13 +120,40 @@ __global__ void k_up2_bwd(int nb, int D, int H, int W, int C, const float* __res
     const int z = (int)(v % D);
     const int b = (int)(v / D);
     const int W2 = 2 * W, H2 = 2 * H, D2 = 2 * D;
-    float s = 0.0f;
+    V s{};
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
         const int xx = 2 * x + (q & 1), yy = 2 * y + ((q >> 1) & 1), zz = 2 * z + (q >> 2);
-        s += dY[((((int64_t)b * D2 + zz) * H2 + yy) * W2 + xx) * C + c];
+        nn_add(s, dY[((((int64_t)b * D2 + zz) * H2 + yy) * W2 + xx) * ld + c]);
     }
     dX[t] = s;
+}
+
+// Y = [A | upsampled X] (fine voxels): the decoder's input in one pass.
+// Bounded by memory: 16 x 32 x 64 x 64 voxels, 32 + 64 channels read 0.17 GB
+// and write 0.40 GB; k_up2 and k_concat wrote and read the upsampled tensor
+// besides (95 us for both).
+template <typename V>
+__global__ void k_up2_concat(int nb, int D, int H, int W, int ca, int cb,
+                             const V* __restrict__ A, const V* __restrict__ X,
+                             V* __restrict__ Y) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int W2 = 2 * W, H2 = 2 * H, D2 = 2 * D, cc = ca + cb;
+    if (t >= (int64_t)nb * D2 * H2 * W2 * cc) return;
+    const int64_t vf = t / cc;
+    const int c = (int)(t - vf * cc);
+    if (c < ca) {
+        Y[t] = A[vf * ca + c];
+        return;
+    }
+    int64_t v = vf;
+    const int x = (int)(v % W2);
+    v /= W2;
+    const int y = (int)(v % H2);
+    v /= H2;
+    const int z = (int)(v % D2);
+    const int b = (int)(v / D2);
+    Y[t] = X[((((int64_t)b * D + z / 2) * H + y / 2) * W + x / 2) * cb + (c - ca)];
 }
 
 // channel concatenation Y = [A | B] (bf16) and its backward split (FP32);
@@ -179,6 +218,33 @@ __global__ void k_bias_grad(int64_t nvox, int C, const float* __restrict__ dZ,
     }
 }
 
+// Block sums of four channels a thread (of lane mod C / 4) added to db: the
+// end of the kernels below, 16 waves a block.
+__device__ __forceinline__ void bias_fold(float s0, float s1, float s2, float s3, int C,
+                                          float (*part)[256], float* __restrict__ db) {
+    const int lanes = C >> 2;  // lanes per channel period
+    for (int sh = 32; sh >= lanes; sh >>= 1) {
+        s0 += __shfl_xor(s0, sh, 64);
+        s1 += __shfl_xor(s1, sh, 64);
+        s2 += __shfl_xor(s2, sh, 64);
+        s3 += __shfl_xor(s3, sh, 64);
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane < lanes) {
+        part[w][4 * lane + 0] = s0;
+        part[w][4 * lane + 1] = s1;
+        part[w][4 * lane + 2] = s2;
+        part[w][4 * lane + 3] = s3;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < C) {
+        float tot = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) tot += part[k][threadIdx.x];
+        atomicAdd(db + threadIdx.x, tot);
+    }
+}
+
 // ReLU backward fused with the bias gradient, for C a multiple of 4 that
 // divides 256 and 16-byte aligned operands.  Each thread takes float4 groups
 // 1024 x gridDim.x apart, so its four channels stay fixed (4 x lane mod C):
@@ -216,45 +282,80 @@ __global__ void __launch_bounds__(1024) k_relu_bias_bwd(int64_t n4, int C,
         s2 += g.z;
         s3 += g.w;
     }
-    const int lanes = C >> 2;  // lanes per channel period
-    for (int sh = 32; sh >= lanes; sh >>= 1) {
-        s0 += __shfl_xor(s0, sh, 64);
-        s1 += __shfl_xor(s1, sh, 64);
-        s2 += __shfl_xor(s2, sh, 64);
-        s3 += __shfl_xor(s3, sh, 64);
+    bias_fold(s0, s1, s2, s3, C, part, db);
+}
+
+// The same for a layer of the network, from where its gradient stands, so
+// that no copy of it is laid out first:
+//   POOL: dA is the gradient of the layer's 2x2x2 average pooling (coarse
+//         voxels, extents D/2, H/2, W/2), an eighth of it for each fine voxel;
+//   dA2:  nullable, the lower C channels of a gradient of ld2 float4 a voxel;
+//   A:    the layer's bf16 output, as the mask (a positive FP32 output that
+//         rounds to a bf16 zero, below 2^-134, counts as zero).
+// Bounded by memory: at 2^21 voxels x 32 channels the pooled form reads 0.44
+// GB and writes 0.13 GB; pool2_bwd, split and k_relu_bias_bwd on the FP32
+// output moved 2.4 GB for it.
+template <bool POOL>
+__global__ void __launch_bounds__(1024) k_relu_bias_net(
+    int64_t n4, int C, unsigned D, unsigned H, unsigned W, const float4* __restrict__ dA,
+    const float4* __restrict__ dA2, int64_t ld2, const uint2* __restrict__ A,
+    uint2* __restrict__ dZb, float* __restrict__ db) {
+    __shared__ float part[16][256];
+    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+    const int lanes = C >> 2, lsh = __ffs(lanes) - 1;  // float4 per voxel, a power of two
+    const int64_t stride = (int64_t)gridDim.x * 1024;
+    for (int64_t t = (int64_t)blockIdx.x * 1024 + threadIdx.x; t < n4; t += stride) {
+        const uint2 h = A[t];
+        const unsigned v = (unsigned)(t >> lsh), c = (unsigned)t & (lanes - 1);
+        float4 g;
+        if (POOL) {
+            const unsigned x = v % W, r = v / W, y = r % H, q = r / H, z = q % D, b = q / D;
+            const int64_t vc =
+                (((int64_t)b * (D / 2) + z / 2) * (H / 2) + y / 2) * (W / 2) + x / 2;
+            g = nn_eighth(dA[(vc << lsh) + c]);
+        } else {
+            g = dA[t];
+        }
+        if (dA2) nn_add(g, dA2[v * ld2 + c]);
+        // positive bf16: 0x0001 .. 0x7f80
+        if ((h.x & 0xffff) - 1u >= 0x7f80u) g.x = 0.0f;
+        if ((h.x >> 16) - 1u >= 0x7f80u) g.y = 0.0f;
+        if ((h.y & 0xffff) - 1u >= 0x7f80u) g.z = 0.0f;
+        if ((h.y >> 16) - 1u >= 0x7f80u) g.w = 0.0f;
+        dZb[t] = make_uint2((uint32_t)nn_f2bf(g.x) | ((uint32_t)nn_f2bf(g.y) << 16),
+                            (uint32_t)nn_f2bf(g.z) | ((uint32_t)nn_f2bf(g.w) << 16));
+        s0 += g.x;
+        s1 += g.y;
+        s2 += g.z;
+        s3 += g.w;
     }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane < lanes) {
-        part[w][4 * lane + 0] = s0;
-        part[w][4 * lane + 1] = s1;
-        part[w][4 * lane + 2] = s2;
-        part[w][4 * lane + 3] = s3;
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < C) {
-        float tot = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) tot += part[k][threadIdx.x];
-        atomicAdd(db + threadIdx.x, tot);
-    }
+    bias_fold(s0, s1, s2, s3, C, part, db);
 }
 
 // Loss on channel 0 of the head output Y (nvox x C): 0.5 mean (Y0 - target)^2
 // summed in FP64 (loss[0] += ...); dY (FP32, nvox x C) = (Y0 - target) / nvox
 // in channel 0 and zero elsewhere
-__global__ void __launch_bounds__(256) k_mse(int64_t nvox, int C, const float* __restrict__ Y,
+// V is float, or float4 with G = C / 4 of them a voxel (a thread each, so the
+// zeros are written in whole lines: 2^21 voxels x 16 channels took 159 us one
+// voxel a thread).
+template <typename V>
+__global__ void __launch_bounds__(256) k_mse(int64_t nvox, int C, int G, const float* __restrict__ Y,
                                              const float* __restrict__ target,
-                                             float* __restrict__ dY, double* __restrict__ loss) {
+                                             V* __restrict__ dY, double* __restrict__ loss) {
     // a grid of at most 1024 blocks; each folds its four waves in LDS and
     // adds once (atomics on one address serialise)
     __shared__ double part[4];
     double l = 0.0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nvox; t += stride) {
-        const float r = Y[t * C] - target[t];
-        l += 0.5 * (double)r * (double)r / (double)nvox;
-        dY[t * C] = r / (float)nvox;
-        for (int c = 1; c < C; ++c) dY[t * C + c] = 0.0f;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nvox * G; t += stride) {
+        const int64_t v = t / G;
+        V o{};
+        if (t == v * G) {
+            const float r = Y[v * C] - target[v];
+            l += 0.5 * (double)r * (double)r / (double)nvox;
+            *(float*)&o = r / (float)nvox;
+        }
+        dY[t] = o;
     }
 #pragma unroll
     for (int sh = 32; sh >= 1; sh >>= 1) l += __shfl_xor(l, sh, 64);
@@ -417,10 +518,30 @@ void launch_nn_up2(int dir, int nb, int D, int H, int W, int C, const void* in, 
         hipLaunchKernelGGL(k_up2<uint16_t>, dim3(nn_blocks(n)), dim3(256), 0, s, nb, D, H, W, C,
                            (const uint16_t*)in, (uint16_t*)out);
     } else {
-        const int64_t n = (int64_t)nb * D * H * W * C;
-        hipLaunchKernelGGL(k_up2_bwd, dim3(nn_blocks(n)), dim3(256), 0, s, nb, D, H, W, C,
-                           (const float*)in, (float*)out);
+        launch_nn_up2_bwd(nb, D, H, W, C, C, (const float*)in, (float*)out, s);
     }
+}
+
+void launch_nn_up2_bwd(int nb, int D, int H, int W, int C, int ld, const float* dY, float* dX,
+                       hipStream_t s) {
+    const int64_t n = (int64_t)nb * D * H * W * C;
+    if (C % 4 == 0 && ld % 4 == 0 && nn_al16(dY) && nn_al16(dX))
+        hipLaunchKernelGGL(k_up2_bwd<float4>, dim3(nn_blocks(n / 4)), dim3(256), 0, s, nb, D, H, W,
+                           C / 4, ld / 4, (const float4*)dY, (float4*)dX);
+    else
+        hipLaunchKernelGGL(k_up2_bwd<float>, dim3(nn_blocks(n)), dim3(256), 0, s, nb, D, H, W, C,
+                           ld, dY, dX);
+}
+
+void launch_nn_up2_concat(int nb, int D, int H, int W, int ca, int cb, const uint16_t* A,
+                          const uint16_t* X, uint16_t* Y, hipStream_t s) {
+    const int64_t n = (int64_t)nb * 8 * D * H * W * (ca + cb);
+    if (ca % 8 == 0 && cb % 8 == 0 && nn_al16(A) && nn_al16(X) && nn_al16(Y))
+        hipLaunchKernelGGL(k_up2_concat<uint4>, dim3(nn_blocks(n / 8)), dim3(256), 0, s, nb, D, H,
+                           W, ca / 8, cb / 8, (const uint4*)A, (const uint4*)X, (uint4*)Y);
+    else
+        hipLaunchKernelGGL(k_up2_concat<uint16_t>, dim3(nn_blocks(n)), dim3(256), 0, s, nb, D, H,
+                           W, ca, cb, A, X, Y);
 }
 
 void launch_nn_concat(int64_t nvox, int ca, int cb, const uint16_t* A, const uint16_t* B,
@@ -462,10 +583,30 @@ void launch_nn_relu_bias_bwd(int64_t nvox, int C, const float* dA, const float* 
                        (uint2*)dZb, db);
 }
 
+void launch_nn_relu_bias_net(const int32_t* shape, const float* dA, int pooled, const float* dA2,
+                             int64_t ld2, const uint16_t* A, uint16_t* dZb, float* db,
+                             hipStream_t s) {
+    const int C = shape[4];
+    const int64_t n4 = (int64_t)shape[0] * shape[1] * shape[2] * shape[3] * C / 4;
+    const dim3 grid((unsigned)std::min<int64_t>((n4 + 1023) / 1024, 512));
+    if (pooled)
+        hipLaunchKernelGGL(k_relu_bias_net<true>, grid, dim3(1024), 0, s, n4, C, shape[1],
+                           shape[2], shape[3], (const float4*)dA, (const float4*)dA2, ld2 / 4,
+                           (const uint2*)A, (uint2*)dZb, db);
+    else
+        hipLaunchKernelGGL(k_relu_bias_net<false>, grid, dim3(1024), 0, s, n4, C, shape[1],
+                           shape[2], shape[3], (const float4*)dA, (const float4*)dA2, ld2 / 4,
+                           (const uint2*)A, (uint2*)dZb, db);
+}
+
 void launch_nn_mse(int64_t nvox, int C, const float* Y, const float* target, float* dY,
                    double* loss, hipStream_t s) {
-    hipLaunchKernelGGL(k_mse, dim3(std::min(nn_blocks(nvox), 1024u)), dim3(256), 0, s, nvox, C, Y,
-                       target, dY, loss);
+    if (C % 4 == 0 && nn_al16(dY))
+        hipLaunchKernelGGL(k_mse<float4>, dim3(std::min(nn_blocks(nvox * (C / 4)), 1024u)),
+                           dim3(256), 0, s, nvox, C, C / 4, Y, target, (float4*)dY, loss);
+    else
+        hipLaunchKernelGGL(k_mse<float>, dim3(std::min(nn_blocks(nvox * C), 1024u)), dim3(256), 0,
+                           s, nvox, C, C, Y, target, dY, loss);
 }
 
 void launch_nn_window_input(const int32_t* n, const float* geo, const float* T, const float* Tface,

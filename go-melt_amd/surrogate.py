@@ -37,24 +37,30 @@ def _check(t, dtype, name):
         raise ValueError(f"{name}: need a contiguous {dtype} tensor on the GPU")
 
 
-def conv3d(X, Wk, bias=None, relu=False, want_bf16=True):
+def conv3d(X, Wk, bias=None, relu=False, want_bf16=True, want_f32=True):
     """Y = conv(X; Wk) + bias (then max(0, .) if relu).  X bf16 (nb,D,H,W,ci),
     Wk bf16 (27, co, ci), bias FP32 (co,) or None.  Returns (Y FP32, Y bf16
-    or None)."""
+    or None); (None, Y bf16) with want_f32 false."""
     _check(X, torch.bfloat16, "X")
     _check(Wk, torch.bfloat16, "Wk")
     co = Wk.shape[1]
     if Wk.shape != (27, co, X.shape[4]):
         raise ValueError("Wk must be (27, cout, cin)")
-    Y = torch.empty(X.shape[:4] + (co,), dtype=torch.float32, device=X.device)
-    Yb = torch.empty_like(Y, dtype=torch.bfloat16) if want_bf16 else None
+    out = X.shape[:4] + (co,)
+    Y = torch.empty(out, dtype=torch.float32, device=X.device) if want_f32 else None
+    Yb = torch.empty(out, dtype=torch.bfloat16, device=X.device) \
+        if want_bf16 or not want_f32 else None
     if bias is not None:
         _check(bias, torch.float32, "bias")
     shape = _shape(X, co)
     nb = C.c_int64()
     N.check(N.lib().gm_conv3d_fwd_ws_bytes(shape, C.byref(nb)))
-    if nb.value > 0:  # few output tiles: the K sum split over blocks
-        ws = torch.empty(nb.value, dtype=torch.uint8, device=X.device)
+    # few output tiles: the K sum split over blocks
+    ws = torch.empty(nb.value, dtype=torch.uint8, device=X.device) if nb.value > 0 else None
+    if not want_f32:
+        N.check(N.lib().gm_conv3d_fwd_bf16(shape, _ptr(X), _ptr(Wk), _ptr(bias), int(relu),
+                                           _ptr(Yb), _ptr(ws), nb.value, _stream()))
+    elif ws is not None:
         N.check(N.lib().gm_conv3d_fwd_ws(shape, _ptr(X), _ptr(Wk), _ptr(bias), int(relu),
                                          _ptr(Y), _ptr(Yb), _ptr(ws), nb.value, _stream()))
     else:
@@ -151,6 +157,33 @@ def up2_bwd(dY):
     return dX
 
 
+def up2_bwd_of(dY, c0):
+    """up2_bwd of the channels from c0 on of an FP32 (nb, 2D, 2H, 2W, ca + C)
+    gradient, without a copy of them."""
+    _check(dY, torch.float32, "dY")
+    nb, D, H, Wd, ld = dY.shape
+    sh = (C.c_int32 * 5)(nb, D // 2, H // 2, Wd // 2, ld - c0)
+    dX = torch.empty((nb, D // 2, H // 2, Wd // 2, ld - c0), dtype=torch.float32,
+                     device=dY.device)
+    N.check(N.lib().gm_nn_up2_bwd(sh, ld, C.c_void_p(dY.data_ptr() + 4 * c0), _ptr(dX),
+                                  _stream()))
+    return dX
+
+
+def up2_concat(A, X):
+    """concat(A, up2(X)) in one pass: bf16 A (nb, 2D, 2H, 2W, ca), X (nb, D, H,
+    W, C)."""
+    _check(A, torch.bfloat16, "A")
+    _check(X, torch.bfloat16, "X")
+    nb, D, H, Wd, cb = X.shape
+    if A.shape[:4] != (nb, 2 * D, 2 * H, 2 * Wd):
+        raise ValueError(f"up2_concat: voxel shapes {tuple(A.shape)} and twice {tuple(X.shape)}")
+    Y = torch.empty(A.shape[:4] + (A.shape[4] + cb,), dtype=torch.bfloat16, device=A.device)
+    N.check(N.lib().gm_nn_up2_concat((C.c_int32 * 5)(nb, D, H, Wd, cb), A.shape[4], _ptr(A),
+                                     _ptr(X), _ptr(Y), _stream()))
+    return Y
+
+
 def concat(A, B):
     if tuple(A.shape[:4]) != tuple(B.shape[:4]):
         raise ValueError(f"concat: voxel shapes {tuple(A.shape)} and {tuple(B.shape)} differ")
@@ -213,6 +246,18 @@ def relu_bias_bwd(dA, A, db, dA2=None):
     return dZb
 
 
+def relu_bias_net(dA, A, db, dA2=None, pooled=False):
+    """relu_bias_bwd of a layer with the bf16 output A: dA the FP32 gradient
+    wrt A, or wrt pool2(A) when pooled; dA2 a gradient whose lower channels
+    are added.  Returns the bf16 dZ."""
+    _check(dA, torch.float32, "dA")
+    dZb = torch.empty_like(A)
+    N.check(N.lib().gm_nn_relu_bias_net((C.c_int32 * 5)(*A.shape), _ptr(dA), int(pooled),
+                                        _ptr(dA2), dA2.shape[4] if dA2 is not None else 0,
+                                        _ptr(A), _ptr(dZb), _ptr(db), _stream()))
+    return dZb
+
+
 def mse(Y, target, loss):
     """loss (FP64 device scalar) += 0.5 mean (Y[..., 0] - target)^2; returns
     the FP32 gradient wrt Y."""
@@ -245,6 +290,12 @@ def mse_energy(Y, target, loss, lam):
 # The operator: a 3-D U-Net of 3x3x3 convolutions
 # ---------------------------------------------------------------------------
 
+def _fused(X, co):
+    """Whether relu_bias_net takes a layer's backward pass: device tensors,
+    a channel count that divides 256, voxel indices of 31 bits."""
+    return X.is_cuda and 256 % co == 0 and X.numel() // X.shape[4] < 1 << 31
+
+
 class Conv:
     """One 3x3x3 convolution layer: FP32 master weights, their bf16 copy,
     FP32 gradients and Adam moments (all device tensors)."""
@@ -261,14 +312,28 @@ class Conv:
         self.moments = [(_zeros(p.shape), _zeros(p.shape)) for p in self.params]
 
     def forward(self, Xb):
+        """bf16 output.  A ReLU layer keeps only that (its FP32 values served
+        as the mask of the backward pass alone: 2^21 voxels x 32 channels
+        write 0.27 GB less here and read 0.13 GB less there), unless the fused
+        backward kernel does not take its shape."""
         self.Xb = Xb
+        if self.relu and _fused(Xb, self.wb.shape[1]):
+            self.A = conv3d(Xb, self.wb, self.b, relu=True, want_f32=False)[1]
+            return self.A
         self.A, Ab = conv3d(Xb, self.wb, self.b, relu=self.relu)
         return Ab
 
-    def backward(self, dA, dA2=None, need_input_grad=True):
-        """dA: FP32 gradient wrt this layer's output; returns the FP32
-        gradient wrt its input (or None)."""
-        dZb = relu_bias_bwd(dA, self.A if self.relu else None, self.grads[1], dA2)
+    def backward(self, dA, skip=None, need_input_grad=True, pooled=False):
+        """dA: FP32 gradient wrt this layer's output (wrt pool2 of it when
+        pooled); skip: a gradient whose lower channels are added to it.
+        Returns the FP32 gradient wrt its input (or None)."""
+        co = self.A.shape[4]
+        if self.relu and _fused(self.Xb, co):
+            dZb = relu_bias_net(dA, self.A, self.grads[1], skip, pooled)
+        else:
+            dA2 = skip if skip is None or skip.shape[4] == co else split(skip, co)[0]
+            dZb = relu_bias_bwd(pool2_bwd(dA) if pooled else dA, self.A if self.relu else None,
+                                self.grads[1], dA2)
         conv3d_bwd_weight(self.Xb, dZb, self.grads[0])
         if not need_input_grad:
             return None
@@ -318,7 +383,7 @@ class UNet:
                 x = pool2(x)
         for k, (c1, c2) in enumerate(self.dec):
             l = len(self.ch) - 2 - k
-            x = concat(self.skips[l], up2(x))
+            x = up2_concat(self.skips[l], x) if x.is_cuda else concat(self.skips[l], up2(x))
             x = c2.forward(c1.forward(x))
         self.head.forward(x)
         return self.head.A
@@ -331,16 +396,13 @@ class UNet:
         for k in reversed(range(len(self.dec))):
             c1, c2 = self.dec[k]
             l = len(self.ch) - 2 - k
-            g = c1.backward(c2.backward(g))
-            ds, du = split(g, self.ch[l])
-            skip_grads[l] = ds
-            g = up2_bwd(du)
-        for l in range(len(self.ch) - 1, -1, -1):
+            g = skip_grads[l] = c1.backward(c2.backward(g))  # [skip | upsampled]
+            g = up2_bwd_of(g, self.ch[l]) if g.is_cuda else up2_bwd(split(g, self.ch[l])[1])
+        last = len(self.ch) - 1
+        for l in range(last, -1, -1):
             c1, c2 = self.enc[l]
-            g2 = c2.backward(g, skip_grads[l]) if l < len(self.ch) - 1 else c2.backward(g)
-            g = c1.backward(g2, need_input_grad=(l > 0))
-            if l > 0:
-                g = pool2_bwd(g)
+            g = c1.backward(c2.backward(g, skip_grads[l], pooled=l < last),
+                            need_input_grad=l > 0)
 
     def step(self, lr=1e-3):
         self.t += 1

@@ -511,6 +511,11 @@ int gm_conv3d_fwd_ws(const int32_t* shape_host, const uint16_t* X, const uint16_
                      const float* bias, int relu, float* Y, uint16_t* Ybf, void* ws,
                      int64_t ws_bytes, void* stream);
 
+/* gm_conv3d_fwd_ws with only the bf16 output (ws nullable). */
+int gm_conv3d_fwd_bf16(const int32_t* shape_host, const uint16_t* X, const uint16_t* Wk,
+                       const float* bias, int relu, uint16_t* Ybf, void* ws, int64_t ws_bytes,
+                       void* stream);
+
 /* Gradient of the input: dX[v][i] = sum_{tap,o} dY[v - s(tap)][o] Wk[tap][o][i]
  * (Wt_work: 27*cin*cout bf16 of caller scratch for the flipped weights). */
 int gm_conv3d_bwd_data(const int32_t* shape_host, const uint16_t* dY, const uint16_t* Wk,
@@ -546,6 +551,14 @@ int gm_nn_concat(int64_t nvox, int ca, int cb, const uint16_t* A, const uint16_t
                  uint16_t* Y, void* stream);
 int gm_nn_split(int64_t nvox, int ca, int cb, const float* dY, float* dA, float* dB,
                 void* stream);
+/* Y = [A | upsampled X] (bf16): gm_nn_up2 and gm_nn_concat in one pass; A has
+ * ca channels on the fine voxels, X coarse_shape's. */
+int gm_nn_up2_concat(const int32_t* coarse_shape_host, int ca, const uint16_t* A,
+                     const uint16_t* X, uint16_t* Y, void* stream);
+/* gm_nn_up2's backward pass from C = coarse_shape[4] channels of a gradient
+ * of ld values a voxel (dY points at the first of them). */
+int gm_nn_up2_bwd(const int32_t* coarse_shape_host, int ld, const float* dY, float* dX,
+                  void* stream);
 /* dZ = (dA + dA2) where A > 0, else 0 (dA2, A nullable); FP32 and a bf16 copy
  * (dZb nullable). */
 int gm_nn_relu_bwd(int64_t n, const float* dA, const float* dA2, const float* A, float* dZ,
@@ -559,6 +572,12 @@ int gm_nn_bias_grad(int64_t nvox, int C, const float* dZ, float* db, void* strea
  * dZb 8-byte aligned.  Sums in a different order from gm_nn_bias_grad. */
 int gm_nn_relu_bias_bwd(int64_t nvox, int C, const float* dA, const float* dA2,
                         const float* A, float* dZ, uint16_t* dZb, float* db, void* stream);
+/* The same for a layer of shape {nb, D, H, W, C} of the network, with its
+ * bf16 output A as the mask and only the bf16 dZb.  pooled: dA is the gradient
+ * of the layer's 2x2x2 average pooling (even extents); dA2 (nullable): the
+ * lower C channels of a gradient of ld2 (multiple of 4) values a voxel. */
+int gm_nn_relu_bias_net(const int32_t* shape_host, const float* dA, int pooled, const float* dA2,
+                        int64_t ld2, const uint16_t* A, uint16_t* dZb, float* db, void* stream);
 /* loss[0] += 0.5 mean_v (Y[v][0] - target[v])^2 (FP64); dY (FP32, nvox x C)
  * = (Y[v][0] - target[v]) / nvox in channel 0, zero elsewhere. */
 int gm_nn_mse(int64_t nvox, int C, const float* Y, const float* target, float* dY,

@@ -165,6 +165,50 @@ def test_relu_bias_fused_rejects(S):
     np.testing.assert_array_equal(_np(dZb), np.ones((10, 48), np.float32))
 
 
+# one block and several, 1 to 64 float4 a voxel, extents off the tile sizes
+@pytest.mark.parametrize("C,cu,shape", [(4, 4, (1, 2, 2, 2)), (16, 16, (2, 6, 10, 14)),
+                                        (32, 64, (3, 16, 34, 30)), (256, 128, (1, 4, 6, 10))])
+def test_network_fused_passes(S, C, cu, shape):
+    """The passes fused over the network's seams against the kernels they
+    join: the same bits, but for the order of the bias sums."""
+    import torch
+    gen = torch.Generator().manual_seed(C + shape[1])
+    nb, D, H, Wd = shape
+    f = lambda *s: torch.randn(s, generator=gen).cuda()
+    A, X = f(nb, D, H, Wd, C).relu().bfloat16(), f(nb, D // 2, H // 2, Wd // 2, cu).bfloat16()
+    np.testing.assert_array_equal(_np(S.up2_concat(A, X)), _np(S.concat(A, S.up2(X))))
+    dC = f(nb, D, H, Wd, C + cu)
+    ds, du = S.split(dC, C)
+    np.testing.assert_array_equal(_np(S.up2_bwd_of(dC, C)), _np(S.up2_bwd(du)))
+    nvox = nb * D * H * Wd
+    for pooled in (False, True):
+        dA = f(nb, D // 2, H // 2, Wd // 2, C) if pooled else f(nb, D, H, Wd, C)
+        for skip, dA2 in ((dC, ds), (None, None)):
+            db, ref = torch.zeros(C).cuda(), torch.zeros(C).cuda()
+            got = S.relu_bias_net(dA, A, db, skip, pooled)
+            want = S.relu_bias_bwd(S.pool2_bwd(dA) if pooled else dA, A.float(), ref, dA2)
+            np.testing.assert_array_equal(_np(got), _np(want))
+            # as test_relu_bias_fused, with up to 512 blocks
+            np.testing.assert_allclose(_np(db), _np(ref), rtol=2e-5,
+                                       atol=512 * 2.0 ** -24 * 4 * np.sqrt(nvox))
+
+
+@pytest.mark.parametrize("shape,ci,co", [((1, 4, 8, 8), 128, 128), ((1, 3, 5, 7), 48, 80),
+                                         ((2, 8, 16, 16), 32, 64), ((1, 4, 6, 10), 16, 32)])
+def test_conv_bf16_output_only(S, shape, ci, co):
+    """want_f32=False (split K sum, general, marching and 16-channel kernels)
+    gives the bf16 output of the full call."""
+    import torch
+    gen = torch.Generator().manual_seed(ci)
+    X = torch.randn(shape + (ci,), generator=gen).bfloat16().cuda()
+    Wk = (0.05 * torch.randn((27, co, ci), generator=gen)).bfloat16().cuda()
+    b = torch.randn(co, generator=gen).cuda()
+    Y, Yb = S.conv3d(X, Wk, b, relu=True)
+    none, got = S.conv3d(X, Wk, b, relu=True, want_f32=False)
+    assert none is None
+    np.testing.assert_array_equal(_np(got), _np(Yb))
+
+
 def test_unet_gradient_direction(S):
     """Directional derivative of the loss through the whole U-Net: the
     kernels' gradient g predicts L(w + e d) - L(w - e d) ~ 2 e <g, d> for a
