@@ -2433,19 +2433,17 @@ static void step_body_general(gm_engine* e, float dt) {
 }
 
 // computeSolutions (cF:2135-2204) as `solutions`, L2 and L3 with the nodal
-// properties of the step's start state (kc_of T2, T3), then the floor at T_amb.
+// properties of the step's start state (kc_of T2, T3), and the floor at T_amb.
+// The faces take the coarse fields before their floor: T1o gets its floor in
+// the L3 launch, T2o's values without it stand in fa2.
 static void solutions_kc(gm_engine* e, const float* V1, const float* V2, float* T1o, float* T2o,
                          float* T3o) {
-    GmStepDesc* d = e->d_desc;
     run_l1(e, V1, T1o, GM_DT_ROW, 0.0f, 0);
-    launch_face_bc(d, 2, 1, e->cfg.level[2], T1o, T1o, e->fa2, e->fb2, e->s);
-    LSArgs a = l2_args_kc(e, e->T2, e->S12, nullptr, V2, 1.0f, T2o, 0);
-    a.clamp = 0;  // the L3 faces take the field before its floor
-    launch_row_step(a, d, e->cfg.level[2], e->d_dm, e->s);
-    launch_face_bc(d, 3, 2, e->cfg.level[3], T2o, T2o, e->fa3, e->fb3, e->s);
-    a = l3_args_kc(e, e->T3, e->S13, nullptr, 0, 1.0f, T3o, nullptr, nullptr);
-    launch_row_step(a, d, e->cfg.level[3], e->d_dm, e->s);
-    launch_clamp2(T1o, e->nn[1], T2o, e->nn[2], e->mat.T_amb, e->s);
+    RowStep r2{l2_args_kc(e, e->T2, e->S12, nullptr, V2, 1.0f, T2o, 0), T1o, e->fa2, nullptr, 0, 0};
+    launch_row_step(r2, e->d_desc, e->cfg.level[2], e->d_dm, e->s);
+    RowStep r3{l3_args_kc(e, e->T3, e->S13, nullptr, 0, 1.0f, T3o, nullptr, nullptr), e->fa2,
+               nullptr, T1o, e->nn[1], 0};
+    launch_row_step(r3, e->d_desc, e->cfg.level[3], e->d_dm, e->s);
 }
 
 // The restrictions of the three pairs of the single step as one launch's

@@ -434,7 +434,15 @@ struct RowPrep {
 void launch_row_prep(RowPrep& a, int64_t nbox, int n3axes, const GmStepDesc* d, const DevMat* m,
                      hipStream_t s);
 // L2 (no srcT) or L3 solve of the single step, kcin from launch_row_state
-void launch_row_step(const LSArgs& a, const GmStepDesc* d, const gm_grid& hg, const DevMat* m,
+struct RowStep {
+    LSArgs a;
+    const float* coarse;  // field of the level above, for the faces
+    float* raw;           // L2: the new field before its floor
+    float* T1;            // field to put the floor on in the same launch
+    int64_t n1;
+    int nbrick;
+};
+void launch_row_step(RowStep& rs, const GmStepDesc* d, const gm_grid& hg, const DevMat* m,
                      hipStream_t s);
 struct RowNodes {
     struct Job {
@@ -447,7 +455,6 @@ struct RowNodes {
     } j[2];  // L1, L2
 };
 void launch_row_nodes(const RowNodes& a, hipStream_t s);
-void launch_clamp2(float* T0, int64_t n0, float* T1, int64_t n1, float Tamb, hipStream_t s);
 struct RowClose {
     const float* T3o;
     float* T3;

@@ -1509,43 +1509,67 @@ void launch_axis_tables(const GmPair* p, int np, const GmStepDesc* d, hipStream_
 // (the x table also carries 6 sqrt(3) P eta).
 // ---------------------------------------------------------------------------
 
+// Entry t / SRC_L of a pair's separable source factors (t: thread index; every
+// lane of a wave takes part, t past the last entry too).  SRC_L lanes share an
+// entry: each evaluates a term (two Gauss points per fine element on both
+// sides of the coarse node) and the group adds them in the order of a single
+// loop.  A loop per thread is a chain of dependent loads and exponentials: 7.6
+// to 11 us for one row or a hundred.
+#define SRC_L 16
 __device__ __forceinline__ void source_table_at(const GmPair& p, const GmStepDesc* __restrict__ d,
                                                 const DevMat& m, int row0, int npos, int use_rows,
                                                 const float* __restrict__ rows_dev,
                                                 float* __restrict__ G, int nmax, int t) {
-    if (t >= npos * 3 * nmax) return;
-    const int A = t % nmax, ax = (t / nmax) % 3, pos = t / (3 * nmax);
+    const int lane = t & (SRC_L - 1);
+    const int i = t / SRC_L;
+    const bool live = i < npos * 3 * nmax;
+    const int A = i % nmax, ax = (i / nmax) % 3, pos = live ? i / (3 * nmax) : 0;
     const GmAxisTab& tb = p.ax[ax];
     const int cmax = p.cmax[ax];
     const int cn = tb.info[1];
-    float s = 0.0f;
-    if (A <= cn) {
-        const float* row = use_rows ? rows_dev + 7 * (row0 + pos) : d->rows[row0 + pos];
-        const float v = row[ax];
-        const float sq = ax == 2 ? m.dsq : m.rsq;
-        const float coef = ax == 2 ? m.dc : m.rc;
-        for (int side = 0; side < 2; ++side) {
-            const int c = A - 1 + side;  // element below (local node 1) / above (node 0)
-            if (c < 0 || c >= cn) continue;
-            const int e0 = tb.info[2 + c], e1 = tb.info[2 + cmax + c];
-            for (int e = e0; e < e1; ++e) {
+    const bool in = live && A <= cn;
+    const float* row = use_rows ? rows_dev + 7 * (row0 + pos) : d->rows[row0 + pos];
+    const float v = row[ax];
+    const float sq = ax == 2 ? m.dsq : m.rsq;
+    const float coef = ax == 2 ? m.dc : m.rc;
+    // fine elements of the coarse element below (local node 1) and above (0)
+    int e0[2] = {0, 0}, n[2] = {0, 0};
 #pragma unroll
-                for (int gg = 0; gg < 2; ++gg) {
-                    const float4 q = tb.q[2 * e + gg];
-                    const float tt = q.x - v;
-                    const float qv = coef * expf((-3.0f * (tt * tt)) / sq);
-                    s += (side == 0 ? q.z : q.y) * qv;
-                }
-            }
-        }
-        if (ax == 0) s *= m.pc6 * row[6];
+    for (int side = 0; side < 2; ++side) {
+        const int c = A - 1 + side;
+        if (!in || c < 0 || c >= cn) continue;
+        e0[side] = tb.info[2 + c];
+        n[side] = 2 * (tb.info[2 + cmax + c] - e0[side]);
     }
-    G[t] = s;
+    const int nt = n[0] + n[1];
+    float s = 0.0f;
+    for (int k0 = 0; __any(k0 < nt); k0 += SRC_L) {
+        const int k = k0 + lane;
+        float w = 0.0f, qv = 0.0f;
+        if (k < nt) {
+            const bool up = k >= n[0];
+            const int kk = up ? k - n[0] : k;
+            const float4 q = tb.q[2 * e0[up] + kk];
+            const float tt = q.x - v;
+            qv = coef * expf((-3.0f * (tt * tt)) / sq);
+            w = up ? q.y : q.z;
+        }
+#pragma unroll
+        for (int j = 0; j < SRC_L; ++j) {
+            const float wj = __shfl(w, j, SRC_L), qj = __shfl(qv, j, SRC_L);
+            if (k0 + j < nt) s += wj * qj;
+        }
+    }
+    if (live && lane == 0) {
+        if (in && ax == 0) s *= m.pc6 * row[6];
+        G[i] = s;
+    }
 }
 
-__global__ void k_source_tables(GmPair p, const GmStepDesc* __restrict__ d, DevMat m, int row0,
-                                int npos, int use_rows, const float* __restrict__ rows_dev,
-                                float* __restrict__ G, int nmax) {
+__global__ void __launch_bounds__(256) k_source_tables(GmPair p, const GmStepDesc* __restrict__ d,
+                                                       DevMat m, int row0, int npos, int use_rows,
+                                                       const float* __restrict__ rows_dev,
+                                                       float* __restrict__ G, int nmax) {
     source_table_at(p, d, m, row0, npos, use_rows, rows_dev, G, nmax,
                     blockIdx.x * blockDim.x + threadIdx.x);
 }
@@ -1553,7 +1577,7 @@ __global__ void k_source_tables(GmPair p, const GmStepDesc* __restrict__ d, DevM
 void launch_source_tables(const GmPair& p, const GmStepDesc* d, const DevMat& m, int row0,
                           int npos, int use_rows, const float* rows_dev, float* G, int nmax,
                           hipStream_t s) {
-    const int n = npos * 3 * nmax;
+    const int n = npos * 3 * nmax * SRC_L;
     hipLaunchKernelGGL(k_source_tables, dim3((n + 255) / 256), dim3(256), 0, s, p, d, m, row0,
                        npos, use_rows, rows_dev, G, nmax);
 }
@@ -3014,8 +3038,8 @@ void launch_melt_single(const GmStepDesc* d, const float* T3, const uint8_t* pre
 // A step is a chain of small kernels, bound by their launches: independent
 // ones share a launch (block ranges), and the whole step is replayed as a
 // graph.  A row with its move took 274 us in 54 launches on 41 x 41 x 21-node
-// levels and 379 us on the part-scale deck (2.06 M L1 nodes), and takes 133
-// and 230 us in 25 recorded ones.
+// levels and 379 us on the part-scale deck (2.06 M L1 nodes), and takes 118
+// and 215 us in 19 (17 of them recorded).
 // ---------------------------------------------------------------------------
 
 // updateStateProperties (cF:2513-2564) of L3 (y = 0: S1, S2, and S2 before
@@ -3073,8 +3097,8 @@ void launch_row_prep(RowPrep& a, int64_t nbox, int n3axes, const GmStepDesc* d, 
                      hipStream_t s) {
     a.b[0] = (int)nblk(nbox);
     a.b[1] = a.b[0] + (int)nblk(a.n_sub1);
-    a.b[2] = a.b[1] + (int)nblk(3 * a.nmax1);
-    a.b[3] = a.b[2] + (int)nblk(3 * a.nmax2);
+    a.b[2] = a.b[1] + (int)nblk(3 * a.nmax1 * SRC_L);
+    a.b[3] = a.b[2] + (int)nblk(3 * a.nmax2 * SRC_L);
     hipLaunchKernelGGL(k_row_prep, dim3(a.b[3] + nblk(n3axes)), dim3(256), 0, s, a, d, m);
 }
 
@@ -3138,31 +3162,6 @@ void launch_row_nodes(const RowNodes& a, hipStream_t s) {
     hipLaunchKernelGGL(k_row_nodes, dim3((n + 255) / 256, 2), dim3(256), 0, s, a);
 }
 
-// Floor at T_amb of two fields (y picks one), 16 bytes at a time.
-__global__ void k_clamp2(float* T0, int64_t n0, float* T1, int64_t n1, float Tamb) {
-    float* T = blockIdx.y ? T1 : T0;
-    const int64_t n = blockIdx.y ? n1 : n0;
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (i + 3 < n) {
-        float4 v = *(const float4*)(T + i);
-        if (v.x < Tamb || v.y < Tamb || v.z < Tamb || v.w < Tamb) {
-            if (v.x < Tamb) v.x = Tamb;
-            if (v.y < Tamb) v.y = Tamb;
-            if (v.z < Tamb) v.z = Tamb;
-            if (v.w < Tamb) v.w = Tamb;
-            *(float4*)(T + i) = v;
-        }
-    } else {
-        for (int64_t k = i; k < n; ++k)
-            if (T[k] < Tamb) T[k] = Tamb;
-    }
-}
-
-void launch_clamp2(float* T0, int64_t n0, float* T1, int64_t n1, float Tamb, hipStream_t s) {
-    hipLaunchKernelGGL(k_clamp2, dim3(nblk((std::max(n0, n1) + 3) / 4), 2), dim3(256), 0, s, T0,
-                       n0, T1, n1, Tamb);
-}
-
 // a * b rounded by itself, never fused into a sum that reads it
 __device__ __forceinline__ float mul_rounded(float a, float b) {
 #pragma clang fp contract(off)
@@ -3174,14 +3173,42 @@ __device__ __forceinline__ float mul_rounded(float a, float b) {
 // and the update in k_level_step's order (k_step_dpp's own form rounds the
 // update differently; over 40 rows the part deck's L2 T' then drifts 3e-5 from
 // the general path, with this form 5e-6).
+// Each wave prolongs the coarse field onto its own face nodes, the field is
+// written with its floor and (L2) without it to raw, for the L3 faces, and
+// blocks past the bricks put the floor on T1: a launch each for these made the
+// two solves of a step five launches longer.
 template <bool SRC, int ZC>
-__global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __restrict__ d,
+__global__ void __launch_bounds__(64) k_row_step(RowStep rs, const GmStepDesc* __restrict__ d,
                                                  const DevMat* __restrict__ m) {
+    const LSArgs& a = rs.a;
+    if ((int)blockIdx.x >= rs.nbrick) {
+        const float Tamb = m->T_amb;
+        const int64_t i0 = ((int64_t)((int)blockIdx.x - rs.nbrick) * 256 + threadIdx.x) * 4;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t i = i0 + 256 * k;
+            float* T = rs.T1 + i;
+            if (i + 3 < rs.n1) {
+                float4 v = *(const float4*)T;
+                if (v.x < Tamb || v.y < Tamb || v.z < Tamb || v.w < Tamb) {
+                    if (v.x < Tamb) v.x = Tamb;
+                    if (v.y < Tamb) v.y = Tamb;
+                    if (v.z < Tamb) v.z = Tamb;
+                    if (v.w < Tamb) v.w = Tamb;
+                    *(float4*)T = v;
+                }
+            } else {
+                for (int64_t j = i; j < rs.n1; ++j)
+                    if (rs.T1[j] < Tamb) rs.T1[j] = Tamb;
+            }
+        }
+        return;
+    }
     const int nx = a.grid.n[0], ny = a.grid.n[1], nz = a.grid.n[2];
     const int nxy = nx * ny, nn = nxy * nz;
     const int nex = nx - 1, ney = ny - 1, nez = nz - 1;
     const int nzc = (nz + ZC - 1) / ZC;
-    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int t = xcd_tile(blockIdx.x, rs.nbrick);
     const int qs = t / nzc, z0 = (t - qs * nzc) * ZC;
     const int lane = (int)threadIdx.x;
     const int q = DXS * qs - 1 + lane;
@@ -3195,7 +3222,6 @@ __global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __r
 
     // ---- loads: planes z0-1 .. z0+ZC, rows y-1 .. y+1 ------------------------
     const auto rT = buf_rsrc(a.T, nb4), rKC = buf_rsrc(a.kcin, 2u * nb4);
-    const auto rFa = buf_rsrc(a.bcA, nb4), rFb = buf_rsrc(a.bcB, nb4);
     float Tw[ZC + 2][3], Kw[ZC + 2][3], Cw[ZC + 2][3];
 #pragma unroll
     for (int p = 0; p < ZC + 2; ++p) {
@@ -3211,7 +3237,8 @@ __global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __r
             Cw[p][r] = buf_ld(rKC, vo, nb4);
         }
     }
-    float corr[ZC], fa[ZC], fb[ZC];
+    const gm_grid& g = d->g[a.level];
+    float corr[ZC], fa[ZC];
     uint32_t oF[ZC];
     bool face[ZC];
 #pragma unroll
@@ -3220,9 +3247,10 @@ __global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __r
         const bool ok = olane && zz < nz;
         face[i] = x == 0 || x == nex || y == 0 || y == ney || zz == 0;
         oF[i] = ok ? 4u * (uint32_t)(base + nxy * i) : GM_OOB;
-        const uint32_t fo = face[i] ? oF[i] : GM_OOB;
-        fa[i] = buf_ld(rFa, fo);
-        fb[i] = buf_ld(rFb, fo);
+        fa[i] = 0.0f;
+        if (ok && face[i])
+            fa[i] = interp_f(d->g[a.level - 1], rs.coarse, coordf(g, 0, x), coordf(g, 1, y),
+                             coordf(g, 2, zz));
         corr[i] = 0.0f;
         if (!SRC) {
             const int bx = x - a.corr_info[0][0], by = y - a.corr_info[1][0],
@@ -3307,7 +3335,7 @@ __global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __r
         }
     }
 
-    const auto rTo = buf_rsrc(a.Tout, nb4);
+    const auto rTo = buf_rsrc(a.Tout, nb4), rRaw = buf_rsrc(SRC ? a.Tout : rs.raw, nb4);
 #pragma unroll
     for (int i = 0; i < ZC; ++i) {
         const float k100 = Ek[i][0], k110 = Ek[i][1];
@@ -3344,23 +3372,23 @@ __global__ void __launch_bounds__(64) k_row_step(LSArgs a, const GmStepDesc* __r
         if (SRC) F = mul_rounded(sx * sy * sz[i], a.w3);
         if (i + 1 == ptop) F += Ftop;
         float Tnew = ((M * Ti - KT) + F + corr[i]) / M;
-        if (face[i]) Tnew = a.alpha * fa[i] + (1.0f - a.alpha) * fb[i];
-        if (a.clamp && Tnew < Tamb) Tnew = Tamb;
+        if (face[i]) Tnew = fa[i];
+        if (!SRC) buf_st(Tnew, rRaw, oF[i]);
+        if (Tnew < Tamb) Tnew = Tamb;
         buf_st(Tnew, rTo, oF[i]);
     }
 }
 
-void launch_row_step(const LSArgs& a0, const GmStepDesc* d, const gm_grid& hg, const DevMat* m,
+void launch_row_step(RowStep& rs, const GmStepDesc* d, const gm_grid& hg, const DevMat* m,
                      hipStream_t s) {
-    LSArgs a = a0;
-    a.grid = hg;
+    rs.a.grid = hg;
     // planes per wave as launch_dpp
-    if (a.srcT)
-        hipLaunchKernelGGL((k_row_step<true, 3>), dim3(batch_bricks(hg, 1, 3)), dim3(64), 0, s, a,
-                           d, m);
+    rs.nbrick = batch_bricks(hg, 1, rs.a.srcT ? 3 : 2);
+    const dim3 g((unsigned)(rs.nbrick + (rs.n1 + 1023) / 1024));
+    if (rs.a.srcT)
+        hipLaunchKernelGGL((k_row_step<true, 3>), g, dim3(64), 0, s, rs, d, m);
     else
-        hipLaunchKernelGGL((k_row_step<false, 2>), dim3(batch_bricks(hg, 1, 2)), dim3(64), 0, s, a,
-                           d, m);
+        hipLaunchKernelGGL((k_row_step<false, 2>), g, dim3(64), 0, s, rs, d, m);
 }
 
 // End of the single step, per L3 node: the new T0, Level0 S1 and the S2
