@@ -177,6 +177,12 @@ def test_network_fused_passes(S, C, cu, shape):
     f = lambda *s: torch.randn(s, generator=gen).cuda()
     A, X = f(nb, D, H, Wd, C).relu().bfloat16(), f(nb, D // 2, H // 2, Wd // 2, cu).bfloat16()
     np.testing.assert_array_equal(_np(S.up2_concat(A, X)), _np(S.concat(A, S.up2(X))))
+    a = _np(A).reshape(nb, D // 2, 2, H // 2, 2, Wd // 2, 2, C)
+    P = np.zeros((nb, D // 2, H // 2, Wd // 2, C), np.float32)
+    for q in range(8):
+        P += a[:, :, q >> 2, :, (q >> 1) & 1, :, q & 1]
+    P = torch.from_numpy(0.125 * P).bfloat16()
+    np.testing.assert_array_equal(_np(S.pool2(A)), _np(P))
     dC = f(nb, D, H, Wd, C + cu)
     ds, du = S.split(dC, C)
     np.testing.assert_array_equal(_np(S.up2_bwd_of(dC, C)), _np(S.up2_bwd(du)))
