@@ -663,8 +663,8 @@ struct gm_engine {
     bool use_graph = true;
     bool graph_ok = false;
     hipGraphExec_t gexec = nullptr;
-    bool row_ok = false;  // the recorded single step (gm_engine_step)
-    hipGraphExec_t row_exec = nullptr;
+    int row_calls = 0;  // single steps since their launches last changed
+    hipGraphExec_t row_exec = nullptr;  // recorded at the GM_ROW_RECORD-th of them
     std::vector<void*> allocs;
 };
 
@@ -705,6 +705,12 @@ extern "C" int gm_engine_destroy(gm_engine* e) {
     }
     delete e;
     return 0;
+}
+
+// the launches' arguments changed: record the graphs again
+static void drop_graphs(gm_engine* e) {
+    e->graph_ok = false;
+    e->row_calls = 0;
 }
 
 static bool pairs_aligned(gm_engine* e);
@@ -932,13 +938,13 @@ extern "C" int gm_engine_set_layer(gm_engine* e, int64_t ne_act, int64_t nn_act,
     e->host.l1_ne_active = ne_act;
     e->host.l1_nn_active = nn_act;
     for (int i = 0; i < 4; ++i) e->host.sub[i] = sub4[i];
-    e->graph_ok = e->row_ok = false;  // static launch arguments changed
+    drop_graphs(e);  // static launch arguments changed
     return 0;
 }
 
 extern "C" int gm_engine_use_graph(gm_engine* e, int enable) {
     e->use_graph = enable != 0;
-    e->graph_ok = e->row_ok = false;
+    drop_graphs(e);
     return 0;
 }
 
@@ -1014,7 +1020,7 @@ extern "C" int gm_engine_load_state(gm_engine* e, const void* host, int64_t byte
         p += a.second;
     }
     // derived state: restriction path and strip layout, descriptor, tables
-    e->graph_ok = e->row_ok = false;
+    drop_graphs(e);
     e->fast_restrict = !pairs_aligned(e);  // force update_alignment to clear partials
     if (update_alignment(e)) return -1;
     if (upload_desc(e, desc_bytes(0))) return -1;
@@ -1031,7 +1037,7 @@ extern "C" int gm_engine_set_accum_mode(gm_engine* e, int external) {
     const bool x = external != 0;
     if (x != e->acc_external) {
         e->acc_external = x;
-        e->graph_ok = e->row_ok = false;  // the recorded step gathers/scatters Level0 or not
+        drop_graphs(e);  // the recorded step gathers/scatters Level0 or not
     }
     return 0;
 }
@@ -1058,7 +1064,7 @@ static int update_alignment(gm_engine* e) {
     const bool a = pairs_aligned(e);
     if (a != e->fast_restrict) {
         e->fast_restrict = a;
-        e->graph_ok = e->row_ok = false;
+        drop_graphs(e);
         for (int i = 0; i < 3; ++i)
             HIPCHK(hipMemsetAsync(e->part[i], 0, pair_elems(e->pair[i].p) * 8 * sizeof(double),
                                   e->s));
@@ -1071,7 +1077,7 @@ static int update_alignment(gm_engine* e) {
         if (R0 != e->strip_R0[i] || a0 != e->strip_a0[i]) {
             e->strip_R0[i] = R0;
             e->strip_a0[i] = a0;
-            e->graph_ok = e->row_ok = false;
+            drop_graphs(e);
         }
     }
     return 0;
@@ -2517,6 +2523,12 @@ static void step_body_aligned(gm_engine* e, RestrictPairs& flux, RestrictPairs& 
     launch_row_close(c, d, e->d_dm, s);
 }
 
+// Calls with the same launches before the step is recorded: a window that moves
+// against L1's nodes changes the restriction's strips (every 50th row of the
+// 41 x 41 x 21-node deck, every row of a faster laser), and recording costs a
+// few direct steps.
+#define GM_ROW_RECORD 8
+
 extern "C" int gm_engine_step(gm_engine* e, const float* row) {
     GmStepDesc& h = e->host;
     h.nrows = 1;
@@ -2529,24 +2541,25 @@ extern "C" int gm_engine_step(gm_engine* e, const float* row) {
         HIPCHK(hipGetLastError());
         return 0;
     }
-    if (!e->use_graph) {
+    if (!e->use_graph || ++e->row_calls < GM_ROW_RECORD) {
         step_body_aligned(e, flux, mass);
         HIPCHK(hipGetLastError());
         return 0;
     }
-    if (!e->row_ok) {
+    if (e->row_calls == GM_ROW_RECORD) {
         if (e->row_exec) {
             HIPCHK(hipGraphExecDestroy(e->row_exec));
             e->row_exec = nullptr;
         }
+        e->row_calls = 0;  // until the graph stands
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(e->s, hipStreamCaptureModeThreadLocal));
         step_body_aligned(e, flux, mass);
         HIPCHK(hipStreamEndCapture(e->s, &g));
         HIPCHK(hipGraphInstantiate(&e->row_exec, g, nullptr, nullptr, 0));
         HIPCHK(hipGraphDestroy(g));
-        e->row_ok = true;
     }
+    e->row_calls = GM_ROW_RECORD;
     HIPCHK(hipGraphLaunch(e->row_exec, e->s));
     return 0;
 }
@@ -2624,7 +2637,7 @@ extern "C" int gm_engine_layer_change(gm_engine* e, int kidx, float new_l1_z0, f
         if (nA > 0) launch_shift_l0(e->L0S1, e->acc, nA, nB, e->nn[0], s);
         HIPCHK(hipMemsetAsync(e->macc, 0, e->nn[0] * 4, s));
     }
-    e->graph_ok = e->row_ok = false;
+    drop_graphs(e);
     if (update_alignment(e)) return -1;
     if (upload_desc(e, desc_bytes(0))) return -1;
     HIPCHK(hipGetLastError());
