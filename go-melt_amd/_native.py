@@ -128,6 +128,7 @@ _SIGS = {
     "gm_engine_move": (_I, [_P, _FP, _FP, _IP]),
     "gm_engine_subcycle": (_I, [_P, _FP, _I]),
     "gm_engine_step": (_I, [_P, _FP]),
+    "gm_engine_step_general": (_I, [_P, _FP]),
     "gm_engine_step_dwell": (_I, [_P, _F]),
     "gm_engine_layer_change": (_I, [_P, _I, _F, _F, _I]),
     "gm_engine_clear_tprime": (_I, [_P]),

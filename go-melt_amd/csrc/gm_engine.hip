@@ -2484,7 +2484,8 @@ static RowNodes row_nodes(gm_engine* e, const float* B1, float* V1, const float*
     return a;
 }
 
-// The single step on node-aligned levels.
+// The single step on node-aligned levels; every field as step_body_general
+// gives it, bit for bit.
 static void step_body_aligned(gm_engine* e, RestrictPairs& flux, RestrictPairs& mass) {
     GmStepDesc* d = e->d_desc;
     hipStream_t s = e->s;
@@ -2529,12 +2530,23 @@ static void step_body_aligned(gm_engine* e, RestrictPairs& flux, RestrictPairs& 
 // few direct steps.
 #define GM_ROW_RECORD 8
 
-extern "C" int gm_engine_step(gm_engine* e, const float* row) {
+static int step_row(gm_engine* e, const float* row) {
     GmStepDesc& h = e->host;
     h.nrows = 1;
     for (int c = 0; c < 7; ++c) h.rows[0][c] = row[c];
     h.dt1 = row[5];
-    if (upload_desc(e, desc_bytes(1))) return -1;
+    return upload_desc(e, desc_bytes(1));
+}
+
+extern "C" int gm_engine_step_general(gm_engine* e, const float* row) {
+    if (step_row(e, row)) return -1;
+    step_body_general(e, row[5]);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+extern "C" int gm_engine_step(gm_engine* e, const float* row) {
+    if (step_row(e, row)) return -1;
     RestrictPairs flux, mass;
     if (!row_restricts(e, true, &flux) || !row_restricts(e, false, &mass)) {
         step_body_general(e, row[5]);

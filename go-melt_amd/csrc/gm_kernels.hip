@@ -186,6 +186,33 @@ __device__ __forceinline__ float src_axis(const gm_grid& g, int d, int i, float 
     return s;
 }
 
+// src_axis with the roundings that k_level_step's block-wide copy of it is
+// compiled to, spelled out: each Gauss point x_a N_a + x_b N_b rounds one
+// product first, on the x axis another one below the node than elsewhere.
+// For kernels whose results are to be k_level_step's bit for bit.
+__device__ __forceinline__ float src_axis_ls(const gm_grid& g, int d, int i, float v, float sq,
+                                             float coef) {
+    float s = 0.0f;
+    const int ne = g.n[d] - 1;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int e = i - 1 + k;
+        if (e < 0 || e >= ne) continue;
+        const float xa = fmaf((float)e, g.h[d], g.x0[d]);
+        const float xb = fmaf((float)(e + 1), g.h[d], g.x0[d]);
+        const int a = i - e;
+#pragma unroll
+        for (int gg = 0; gg < 2; ++gg) {
+            const float na = gg == 0 ? GA : GB, nb = gg == 0 ? GB : GA;
+            const float xq = d == 0 && k == 0 ? fmaf(xb, nb, xa * na) : fmaf(xa, na, xb * nb);
+            const float t = xq - v;
+            const float qv = coef * expf((-3.0f * (t * t)) / sq);
+            s = fmaf(a == gg ? GA : GB, qv, s);
+        }
+    }
+    return s;
+}
+
 // floor(u / R) for 0 <= u < 2^20 from a reciprocal of R (rcp error far below
 // the 0.5 / R distance of (u + 0.5) / R from an integer)
 __device__ __forceinline__ int fdiv_small(int u, float invR) {
@@ -1288,6 +1315,8 @@ void launch_copy_multi(const CopyList& L, int n, hipStream_t s) {
 
 // Separable source factors of every L3 node line for the desc rows:
 // src_axis of x (times 6 sqrt(3) eta P w3), y and z (cF:1013-1025, 2986-3010).
+// LS: as k_level_step evaluates them.
+template <bool LS>
 __device__ __forceinline__ void src3_table_at(const GmStepDesc* __restrict__ d,
                                               const DevMat* __restrict__ m, int nrows, float w3,
                                               float* __restrict__ out, int t) {
@@ -1296,20 +1325,21 @@ __device__ __forceinline__ void src3_table_at(const GmStepDesc* __restrict__ d,
     if (t >= nrows * n) return;
     const int r = t / n, i = t % n;
     const float* row = d->rows[r];
+    const auto ax = LS ? src_axis_ls : src_axis;
     float v;
     if (i < g.n[0]) {
-        v = src_axis(g, 0, i, row[0], m->rsq, m->rc) * (m->pc6 * row[6] * w3);
+        v = ax(g, 0, i, row[0], m->rsq, m->rc) * (m->pc6 * row[6] * w3);
     } else if (i < g.n[0] + g.n[1]) {
-        v = src_axis(g, 1, i - g.n[0], row[1], m->rsq, m->rc);
+        v = ax(g, 1, i - g.n[0], row[1], m->rsq, m->rc);
     } else {
-        v = src_axis(g, 2, i - g.n[0] - g.n[1], row[2], m->dsq, m->dc);
+        v = ax(g, 2, i - g.n[0] - g.n[1], row[2], m->dsq, m->dc);
     }
     out[t] = v;
 }
 
 __global__ void k_src3_tables(const GmStepDesc* __restrict__ d, const DevMat* __restrict__ m,
                               int nrows, float w3, float* __restrict__ out) {
-    src3_table_at(d, m, nrows, w3, out, blockIdx.x * blockDim.x + threadIdx.x);
+    src3_table_at<false>(d, m, nrows, w3, out, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 void launch_src3_tables(const GmStepDesc* d, const DevMat* m, int nrows, int ntot, float w3,
@@ -3103,7 +3133,7 @@ __global__ void __launch_bounds__(256) k_row_prep(RowPrep a, const GmStepDesc* _
     } else if (b < a.b[3]) {
         source_table_at(a.p2, d, *m, 0, 1, 0, nullptr, a.G2, a.nmax2, (b - a.b[2]) * 256 + t);
     } else {
-        src3_table_at(d, m, 1, 1.0f, a.src3, (b - a.b[3]) * 256 + t);
+        src3_table_at<true>(d, m, 1, 1.0f, a.src3, (b - a.b[3]) * 256 + t);
     }
 }
 
@@ -3183,10 +3213,13 @@ __device__ __forceinline__ float mul_rounded(float a, float b) {
 }
 
 // Fine-level (L2, L3) solve of the single step on the nodal k, cp of
-// k_row_state: k_step_dpp's wave layout and neighbour access, with the sums
-// and the update in k_level_step's order (k_step_dpp's own form rounds the
-// update differently; over 40 rows the part deck's L2 T' then drifts 3e-5 from
-// the general path, with this form 5e-6).
+// k_row_state: k_step_dpp's wave layout and neighbour access, with
+// k_level_step's sums and update, rounding by rounding (k_step_dpp's own form
+// of the update leaves the part deck's L2 T' 2.6e-5 off after 40 rows).  The
+// top flux and the source factors (src_axis_ls) name the products that are
+// rounded; left to the compiler they were others than in k_level_step, which
+// moved 85 of 520,251 L3 nodes by a rounding in one row of the part deck and
+// its L3 T' by 2.6e-3 over many.
 // Each wave prolongs the coarse field onto its own face nodes, the field is
 // written with its floor and (L2) without it to raw, for the L3 faces, and
 // blocks past the bricks put the floor on T1: a launch each for these made the
@@ -3333,7 +3366,11 @@ __global__ void __launch_bounds__(64) k_row_step(RowStep rs, const GmStepDesc* _
             const bool ok = ein && ey >= 0 && ey < ney;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const float Tq = n2(g, 0) * t0 + n2(g, 1) * t1 + n2(g, 2) * t2 + n2(g, 3) * t3;
+                // the products that k_level_step rounds: n2(g, 1) t1 of the even
+                // points, n2(g, 0) t0 of the odd ones
+                float Tq = g & 1 ? fmaf(n2(g, 1), t1, n2(g, 0) * t0)
+                                 : fmaf(n2(g, 0), t0, n2(g, 1) * t1);
+                Tq = fmaf(n2(g, 3), t3, fmaf(n2(g, 2), t2, Tq));
                 Fq[r][g] = ok ? face_flux(*m, Tq) * a.w2 : 0.0f;
             }
         }

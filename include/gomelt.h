@@ -367,6 +367,10 @@ int gm_multi_destroy(gm_multi* m);
  * see gm_engine_set_accum_mode) it also applies the single-step driver's
  * melt-time bookkeeping (go_melt.py:339-357) to the Level0 maps. */
 int gm_engine_step(gm_engine* e, const float* row_host);
+/* gm_engine_step by the kernels of levels that are not node-aligned, launched
+ * one by one.  On node-aligned levels gm_engine_step takes merged kernels;
+ * both give the same bits. */
+int gm_engine_step_general(gm_engine* e, const float* row_host);
 
 /* Engine state for the driver's per-layer checkpoint (go_melt.py:390-411)
  * and its resume (go_melt.py:115-129): every persistent array of the three

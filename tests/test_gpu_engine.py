@@ -140,6 +140,57 @@ def test_single_steps_vs_oracle(oracle, tmp_path, n, dt3, track):
         assert _relT(a, b) < 5e-4, (k, _relT(a, b))
 
 
+# the track deck's hot pool (source and top flux), property tables on planes
+# smaller than a lane strip, tables without per-bin records, and L3 nodes past
+# 2^20 (k_level_step's 8-plane blocks)
+@pytest.mark.parametrize("deck", ["track", "strip", "close", "large"])
+def test_single_step_routes_equal(tmp_path, deck):
+    """gm_engine_step's merged kernels (direct and recorded) against
+    gm_engine_step_general from the same states: every byte of the engine's
+    state and of the Level0 melt-time maps."""
+    import json
+    import _native as N
+    import computeFunctions as cf
+    import go_melt as G
+    if deck == "track":
+        inp, g = W.single_track()
+    else:
+        n, dt, track = {"strip": ((60, 4, 2), 1e-5, 0.03), "close": ((36, 20, 12), 1e-5, 0.03),
+                        "large": ((130, 96, 92), 1e-6, 0.02)}[deck]
+        k, cp = (CLOSE_K, CLOSE_CP) if deck == "close" else (W.K_TABLE, W.CP_TABLE)
+        inp, g = W.tiny(n=n, n2=2, n3=3, track=track, dt3=dt,
+                        props={"laser_power": 900.0, "emissivity": 0.4, "laser_radius": 0.1,
+                               "laser_depth": 0.1, "thermal_conductivity_bulk_table": k,
+                               "heat_capacity_solid_table": cp})
+    with open(W.write_deck(inp, g, str(tmp_path))) as fh:
+        run = G.TimeLoop(json.load(fh), quiet=True, write_outputs=False)
+    run.step_chunk(next(run.chunks()))
+    maps = [run.Levels[0][k] for k in ("accum_time", "max_accum_time")]
+    rows = [r for c in run.chunks() for r in c][:12]
+    for i, pos in enumerate(rows):  # the graph is recorded within them
+        run.Levels, run.Shapes, run.LInterp, run.move_hist = cf.moveEverything(
+            pos, run.laser_start, run.Levels, run.move_hist, run.LInterp, run.eng.r12,
+            run.eng.r23, run.Properties["layer_height"])
+        row = np.asarray(pos, np.float32)
+        compare = i in (0, 1, len(rows) - 1)
+        if compare:
+            run.eng.sync()
+            acc0 = [m.numpy() for m in maps]
+            state = run.eng.save_state()
+        N.check(N.lib().gm_engine_step(run.eng.h, N.fptr(row)))
+        if not compare:
+            continue
+        got = run.eng.save_state(), [m.numpy() for m in maps]
+        run.eng.load_state(state)
+        for m, a in zip(maps, acc0):
+            m.upload(a)
+        N.check(N.lib().gm_engine_step_general(run.eng.h, N.fptr(row)))
+        want = run.eng.save_state(), [m.numpy() for m in maps]
+        assert got[0] == want[0], (deck, i)
+        for a, b in zip(got[1], want[1]):
+            np.testing.assert_array_equal(a, b)
+
+
 def test_driver_vs_oracle_unaligned_windows(oracle, tmp_path):
     """L2 origin a quarter of an L1 spacing off the L1 nodes: the coarse
     overlap nodes are not fine nodes, so the engine takes the general
