@@ -162,6 +162,8 @@ def up2_bwd_of(dY, c0):
     gradient, without a copy of them."""
     _check(dY, torch.float32, "dY")
     nb, D, H, Wd, ld = dY.shape
+    if D % 2 or H % 2 or Wd % 2 or not 0 <= c0 < ld:
+        raise ValueError(f"up2_bwd_of: even extents and a channel of {tuple(dY.shape)}, not {c0}")
     sh = (C.c_int32 * 5)(nb, D // 2, H // 2, Wd // 2, ld - c0)
     dX = torch.empty((nb, D // 2, H // 2, Wd // 2, ld - c0), dtype=torch.float32,
                      device=dY.device)
@@ -251,6 +253,22 @@ def relu_bias_net(dA, A, db, dA2=None, pooled=False):
     wrt A, or wrt pool2(A) when pooled; dA2 a gradient whose lower channels
     are added.  Returns the bf16 dZ."""
     _check(dA, torch.float32, "dA")
+    _check(A, torch.bfloat16, "A")
+    _check(db, torch.float32, "db")
+    # the kernel indexes every operand by A's shape
+    nb, D, H, Wd, nc = A.shape
+    if pooled and (D % 2 or H % 2 or Wd % 2):
+        raise ValueError("relu_bias_net: a pooled gradient needs even extents")
+    want = (nb, D // 2, H // 2, Wd // 2, nc) if pooled else (nb, D, H, Wd, nc)
+    if tuple(dA.shape) != want:
+        raise ValueError(f"relu_bias_net: gradient {tuple(dA.shape)}, need {want}")
+    if db.numel() != nc:
+        raise ValueError("relu_bias_net: one bias per channel")
+    if dA2 is not None:
+        _check(dA2, torch.float32, "dA2")
+        if tuple(dA2.shape[:4]) != (nb, D, H, Wd) or dA2.dim() != 5 or dA2.shape[4] < nc:
+            raise ValueError(f"relu_bias_net: added gradient {tuple(dA2.shape)} on "
+                             f"{tuple(A.shape)}")
     dZb = torch.empty_like(A)
     N.check(N.lib().gm_nn_relu_bias_net((C.c_int32 * 5)(*A.shape), _ptr(dA), int(pooled),
                                         _ptr(dA2), dA2.shape[4] if dA2 is not None else 0,

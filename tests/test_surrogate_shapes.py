@@ -84,3 +84,53 @@ def test_unet_pass_shapes(monkeypatch, channels, window):
     Y = net.forward(X)
     assert Y.shape == (2,) + window + (16,)
     net.backward(torch.empty(Y.shape))
+
+
+def test_seam_wrappers_check_their_operands(monkeypatch):
+    """relu_bias_net and up2_bwd_of hand raw pointers to kernels that index
+    every operand by one shape: operands of other shapes, dtypes or strides
+    are refused before a launch (CPU tensors, a library that records it)."""
+    torch = pytest.importorskip("torch")
+    import surrogate as S
+
+    class Lib:
+        launched = 0
+
+        def __getattr__(self, name):
+            def call(*a):
+                self.launched += 1
+                return 0
+            return call
+
+    lib = Lib()
+    monkeypatch.setattr(S.N, "lib", lambda: lib)
+    monkeypatch.setattr(S, "_stream", lambda: None)
+
+    def check(t, dtype, name):  # S._check, but for the device
+        if t.dtype != dtype or not t.is_contiguous():
+            raise ValueError(name)
+
+    monkeypatch.setattr(S, "_check", check)
+    f = lambda *s: torch.zeros(s)  # noqa: E731
+    A = f(2, 4, 6, 8, 32).bfloat16()
+    dA, half, wide, db = f(2, 4, 6, 8, 32), f(2, 2, 3, 4, 32), f(2, 4, 6, 8, 96), f(32)
+    for k, ok in enumerate([(dA, A, db), (dA, A, db, dA), (dA, A, db, wide),
+                            (half, A, db, wide, True), (half, A, db, None, True)]):
+        S.relu_bias_net(*ok)
+        assert lib.launched == k + 1
+    odd = f(1, 3, 4, 4, 16)
+    lib.launched = 0
+    for bad in [(half, A, db), (dA, A, db, None, True), (f(1, 4, 6, 8, 32), A, db),
+                (f(2, 4, 6, 8, 16), A, db), (f(2 * 4 * 6 * 8 * 32), A, db),
+                (dA, A.float(), db), (dA, A.transpose(2, 3), db), (dA, A, f(16)),
+                (dA, A, db.double()), (dA, A, db, half), (dA, A, db, f(2, 4, 6, 8, 16)),
+                (dA, A, db, wide.bfloat16()), (dA, A, db, wide[..., :64]),
+                (dA, A, db, f(2, 4, 6, 8)), (half, A, db, half, True),
+                (f(1, 1, 2, 2, 16), odd.bfloat16(), f(16), None, True)]:
+        with pytest.raises(ValueError):
+            S.relu_bias_net(*bad)
+    for dY, c0 in [(wide, 96), (wide, -1), (wide, 200), (odd, 0), (wide[..., 32:], 0)]:
+        with pytest.raises(ValueError):
+            S.up2_bwd_of(dY, c0)
+    assert lib.launched == 0
+    assert S.up2_bwd_of(wide, 32).shape == (2, 2, 3, 4, 64) and lib.launched == 1
