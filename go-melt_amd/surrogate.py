@@ -309,9 +309,9 @@ def mse_energy(Y, target, loss, lam):
 # ---------------------------------------------------------------------------
 
 def _fused(X, co):
-    """Whether relu_bias_net takes a layer's backward pass: device tensors,
-    a channel count that divides 256, voxel indices of 31 bits."""
-    return X.is_cuda and 256 % co == 0 and X.numel() // X.shape[4] < 1 << 31
+    """Whether relu_bias_net takes a layer's backward pass: a channel count
+    that divides 256, voxel indices of 31 bits."""
+    return 256 % co == 0 and X.numel() // X.shape[4] < 1 << 31
 
 
 class Conv:
@@ -401,8 +401,7 @@ class UNet:
                 x = pool2(x)
         for k, (c1, c2) in enumerate(self.dec):
             l = len(self.ch) - 2 - k
-            x = up2_concat(self.skips[l], x) if x.is_cuda else concat(self.skips[l], up2(x))
-            x = c2.forward(c1.forward(x))
+            x = c2.forward(c1.forward(up2_concat(self.skips[l], x)))
         self.head.forward(x)
         return self.head.A
 
@@ -415,7 +414,7 @@ class UNet:
             c1, c2 = self.dec[k]
             l = len(self.ch) - 2 - k
             g = skip_grads[l] = c1.backward(c2.backward(g))  # [skip | upsampled]
-            g = up2_bwd_of(g, self.ch[l]) if g.is_cuda else up2_bwd(split(g, self.ch[l])[1])
+            g = up2_bwd_of(g, self.ch[l])
         last = len(self.ch) - 1
         for l in range(last, -1, -1):
             c1, c2 = self.enc[l]

@@ -9,12 +9,13 @@ class _Shapes:
 
     def __init__(self, torch):
         self.t = torch
+        self.seams = 0  # fused passes taken
 
-    def conv3d(self, X, Wk, bias=None, relu=False, want_bf16=True):
+    def conv3d(self, X, Wk, bias=None, relu=False, want_bf16=True, want_f32=True):
         assert X.dim() == 5 and Wk.shape == (27, Wk.shape[1], X.shape[4]), (X.shape, Wk.shape)
         assert X.shape[4] % 16 == 0 and Wk.shape[1] % 16 == 0
         Y = self.t.empty(X.shape[:4] + (Wk.shape[1],))
-        return Y, Y.to(self.t.bfloat16)
+        return Y if want_f32 else None, Y.to(self.t.bfloat16)
 
     def conv3d_bwd_data(self, dY, Wk, want_bf16=True):
         assert dY.shape[4] == Wk.shape[1]
@@ -36,6 +37,13 @@ class _Shapes:
         self.bias_grad(dA, db)
         return self.relu_bwd(dA, A, dA2)[1]
 
+    def relu_bias_net(self, dA, A, db, dA2=None, pooled=False):
+        assert A.dtype == self.t.bfloat16 and db.numel() == A.shape[-1]
+        assert (self.pool2(A) if pooled else A).shape == dA.shape, (A.shape, dA.shape)
+        assert dA2 is None or (dA2.shape[:4] == A.shape[:4] and dA2.shape[4] >= A.shape[4])
+        self.seams += 1
+        return self.t.empty(A.shape)
+
     def pool2(self, X):
         assert all(s % 2 == 0 for s in X.shape[1:4])
         return self.t.empty(X.shape[:1] + tuple(s // 2 for s in X.shape[1:4]) + X.shape[4:])
@@ -47,6 +55,15 @@ class _Shapes:
 
     def up2_bwd(self, dY):
         return self.pool2(dY)
+
+    def up2_bwd_of(self, dY, c0):
+        assert 0 < c0 < dY.shape[4]
+        self.seams += 1
+        return self.pool2(dY[..., c0:])
+
+    def up2_concat(self, A, X):
+        self.seams += 1
+        return self.concat(A, self.up2(X))
 
     def concat(self, A, B):
         assert A.shape[:4] == B.shape[:4], (A.shape, B.shape)
@@ -75,7 +92,7 @@ def test_unet_pass_shapes(monkeypatch, channels, window):
     f = _Shapes(torch)
     for name in ("conv3d", "conv3d_bwd_data", "conv3d_bwd_weight", "relu_bwd", "bias_grad",
                  "relu_bias_bwd", "pool2", "pool2_bwd", "up2", "up2_bwd", "concat", "split", "mse",
-                 "to_bf16"):
+                 "to_bf16", "relu_bias_net", "up2_bwd_of", "up2_concat"):
         monkeypatch.setattr(S, name, getattr(f, name))
     monkeypatch.setattr(S, "_zeros", f.zeros)
     monkeypatch.setattr(torch.Tensor, "cuda", lambda self, *a, **k: self)
@@ -84,6 +101,9 @@ def test_unet_pass_shapes(monkeypatch, channels, window):
     Y = net.forward(X)
     assert Y.shape == (2,) + window + (16,)
     net.backward(torch.empty(Y.shape))
+    # the passes a device runs: two seams a decoder level, a backward pass a
+    # layer but the head
+    assert f.seams == 2 * (len(channels) - 1) + len(net.layers()) - 1
 
 
 def test_seam_wrappers_check_their_operands(monkeypatch):
