@@ -248,6 +248,15 @@ def relu_bias_bwd(dA, A, db, dA2=None):
     return dZb
 
 
+def _aligned(t):
+    """t, or a copy of it where it does not start on 16 bytes."""
+    if t is None or t.data_ptr() % 16 == 0:
+        return t
+    c = torch.empty_like(t)
+    N.check(N.lib().gm_memcpy_d2d(_ptr(c), _ptr(t), t.numel() * t.element_size(), _stream()))
+    return c
+
+
 def relu_bias_net(dA, A, db, dA2=None, pooled=False):
     """relu_bias_bwd of a layer with the bf16 output A: dA the FP32 gradient
     wrt A, or wrt pool2(A) when pooled; dA2 a gradient whose lower channels
@@ -269,6 +278,7 @@ def relu_bias_net(dA, A, db, dA2=None, pooled=False):
         if tuple(dA2.shape[:4]) != (nb, D, H, Wd) or dA2.dim() != 5 or dA2.shape[4] < nc:
             raise ValueError(f"relu_bias_net: added gradient {tuple(dA2.shape)} on "
                              f"{tuple(A.shape)}")
+    dA, dA2 = _aligned(dA), _aligned(dA2)
     dZb = torch.empty_like(A)
     N.check(N.lib().gm_nn_relu_bias_net((C.c_int32 * 5)(*A.shape), _ptr(dA), int(pooled),
                                         _ptr(dA2), dA2.shape[4] if dA2 is not None else 0,
@@ -341,15 +351,15 @@ class Conv:
         self.A, Ab = conv3d(Xb, self.wb, self.b, relu=self.relu)
         return Ab
 
-    def backward(self, dA, skip=None, need_input_grad=True, pooled=False):
+    def backward(self, dA, dA2=None, need_input_grad=True, pooled=False):
         """dA: FP32 gradient wrt this layer's output (wrt pool2 of it when
-        pooled); skip: a gradient whose lower channels are added to it.
+        pooled); dA2: a gradient whose lower channels are added to it.
         Returns the FP32 gradient wrt its input (or None)."""
         co = self.A.shape[4]
         if self.relu and _fused(self.Xb, co):
-            dZb = relu_bias_net(dA, self.A, self.grads[1], skip, pooled)
+            dZb = relu_bias_net(dA, self.A, self.grads[1], dA2, pooled)
         else:
-            dA2 = skip if skip is None or skip.shape[4] == co else split(skip, co)[0]
+            dA2 = dA2 if dA2 is None or dA2.shape[4] == co else split(dA2, co)[0]
             dZb = relu_bias_bwd(pool2_bwd(dA) if pooled else dA, self.A if self.relu else None,
                                 self.grads[1], dA2)
         conv3d_bwd_weight(self.Xb, dZb, self.grads[0])

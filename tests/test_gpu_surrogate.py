@@ -199,6 +199,28 @@ def test_network_fused_passes(S, C, cu, shape):
                                        atol=512 * 2.0 ** -24 * 4 * np.sqrt(nvox))
 
 
+def test_layer_backward_unaligned_gradients(S):
+    """A layer's backward pass takes gradients that start off 16 bytes, the
+    second one by name: the results of aligned copies, but for the order of
+    the bias sums (512 blocks at most, unit values)."""
+    import torch
+    gen = torch.Generator().manual_seed(3)
+    c = S.Conv(16, 32, True, gen)
+    c.forward(torch.randn((1, 4, 6, 10, 16), generator=gen).bfloat16().cuda())
+    sh = (1, 4, 6, 10, 32)
+    off = lambda: torch.randn(240 * 32 + 1, generator=gen).cuda()[1:].view(sh)  # noqa: E731
+    dA, dA2 = off(), off()
+    assert dA.data_ptr() % 16 == 4 and dA.is_contiguous()
+    got = [c.backward(dA, dA2=dA2)] + [g.clone() for g in c.grads]
+    for g in c.grads:
+        S.zero(g)
+    want = [c.backward(dA.clone(), dA2.clone())] + c.grads
+    np.testing.assert_array_equal(_np(got[0]), _np(want[0]))
+    # FP32 sums in no fixed order: see test_relu_bias_fused
+    for a, b in zip(got[1:], want[1:]):
+        np.testing.assert_allclose(_np(a), _np(b), rtol=2e-5, atol=512 * 2.0 ** -24 * 4 * 240 ** 0.5)
+
+
 @pytest.mark.parametrize("shape,ci,co", [((1, 4, 8, 8), 128, 128), ((1, 3, 5, 7), 48, 80),
                                          ((2, 8, 16, 16), 32, 64), ((1, 4, 6, 10), 16, 32)])
 def test_conv_bf16_output_only(S, shape, ci, co):
