@@ -346,18 +346,27 @@ class Conv:
         backward kernel does not take its shape."""
         self.Xb = Xb
         if self.relu and _fused(Xb, self.wb.shape[1]):
-            self.A = conv3d(Xb, self.wb, self.b, relu=True, want_f32=False)[1]
-            return self.A
-        self.A, Ab = conv3d(Xb, self.wb, self.b, relu=self.relu)
+            self._A, self.mask = None, conv3d(Xb, self.wb, self.b, relu=True, want_f32=False)[1]
+            return self.mask
+        self._A, Ab = conv3d(Xb, self.wb, self.b, relu=self.relu)
         return Ab
+
+    @property
+    def A(self):
+        """FP32 output of the last forward pass.  Where only the bf16 output
+        was kept, the first read evaluates the layer again, on its input and
+        the weights as they are then (before a step: those of the pass)."""
+        if self._A is None:
+            self._A = conv3d(self.Xb, self.wb, self.b, relu=True, want_bf16=False)[0]
+        return self._A
 
     def backward(self, dA, dA2=None, need_input_grad=True, pooled=False):
         """dA: FP32 gradient wrt this layer's output (wrt pool2 of it when
         pooled); dA2: a gradient whose lower channels are added to it.
         Returns the FP32 gradient wrt its input (or None)."""
-        co = self.A.shape[4]
+        co = self.wb.shape[1]
         if self.relu and _fused(self.Xb, co):
-            dZb = relu_bias_net(dA, self.A, self.grads[1], dA2, pooled)
+            dZb = relu_bias_net(dA, self.mask, self.grads[1], dA2, pooled)
         else:
             dA2 = dA2 if dA2 is None or dA2.shape[4] == co else split(dA2, co)[0]
             dZb = relu_bias_bwd(pool2_bwd(dA) if pooled else dA, self.A if self.relu else None,

@@ -221,6 +221,25 @@ def test_layer_backward_unaligned_gradients(S):
         np.testing.assert_allclose(_np(a), _np(b), rtol=2e-5, atol=512 * 2.0 ** -24 * 4 * 240 ** 0.5)
 
 
+def test_layer_output_reads_fp32(S):
+    """Conv.A of a hidden layer: the FP32 output of its forward pass, though
+    that keeps the bf16 one."""
+    import torch
+    gen = torch.Generator().manual_seed(5)
+    c = S.Conv(32, 48, True, gen)      # separate backward passes
+    d = S.Conv(48, 64, True, gen)      # fused
+    x = torch.randn((1, 4, 8, 10, 32), generator=gen).bfloat16().cuda()
+    y = c.forward(x)
+    z = d.forward(y)
+    for layer, xin, out in ((c, x, y), (d, y, z)):
+        Y, Yb = S.conv3d(xin, layer.wb, layer.b, relu=True)
+        assert layer.A.dtype == torch.float32
+        np.testing.assert_array_equal(_np(layer.A), _np(Y))
+        np.testing.assert_array_equal(_np(out), _np(Yb))
+    z = d.forward(y * 2)               # a new pass, new values
+    np.testing.assert_array_equal(_np(d.A.bfloat16()), _np(z))
+
+
 @pytest.mark.parametrize("shape,ci,co", [((1, 4, 8, 8), 128, 128), ((1, 3, 5, 7), 48, 80),
                                          ((2, 8, 16, 16), 32, 64), ((1, 4, 6, 10), 16, 32)])
 def test_conv_bf16_output_only(S, shape, ci, co):
