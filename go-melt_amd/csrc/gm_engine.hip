@@ -7,6 +7,7 @@
 // that is uploaded once per call; every kernel reads the moving meshes from
 // that descriptor, so the ~330 launches of a subcycled L1 step are recorded
 // once into a hipGraph and replayed for every later step.
+#include <limits.h>
 #include <math.h>
 #include <string.h>
 
@@ -2530,6 +2531,31 @@ static void step_body_aligned(gm_engine* e, RestrictPairs& flux, RestrictPairs& 
 // few direct steps.
 #define GM_ROW_RECORD 8
 
+// Whether this step replays its recorded graph, which is recorded at the
+// GM_ROW_RECORD-th call.  The null stream takes no capture; where a recording
+// fails, the launches go on one by one until they change.
+static bool row_graph(gm_engine* e, RestrictPairs& flux, RestrictPairs& mass) {
+    if (!e->use_graph || !e->s || ++e->row_calls < GM_ROW_RECORD) return false;
+    if (e->row_calls > GM_ROW_RECORD) {
+        e->row_calls = GM_ROW_RECORD + 1;
+        return true;
+    }
+    if (e->row_exec) (void)hipGraphExecDestroy(e->row_exec);
+    e->row_exec = nullptr;
+    hipGraph_t g = nullptr;
+    if (hipStreamBeginCapture(e->s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+        step_body_aligned(e, flux, mass);
+        if (hipStreamEndCapture(e->s, &g) != hipSuccess ||
+            hipGraphInstantiate(&e->row_exec, g, nullptr, nullptr, 0) != hipSuccess)
+            e->row_exec = nullptr;
+        if (g) (void)hipGraphDestroy(g);
+    }
+    if (e->row_exec) return true;
+    (void)hipGetLastError();
+    e->row_calls = INT_MIN;
+    return false;
+}
+
 static int step_row(gm_engine* e, const float* row) {
     GmStepDesc& h = e->host;
     h.nrows = 1;
@@ -2553,26 +2579,12 @@ extern "C" int gm_engine_step(gm_engine* e, const float* row) {
         HIPCHK(hipGetLastError());
         return 0;
     }
-    if (!e->use_graph || ++e->row_calls < GM_ROW_RECORD) {
+    if (row_graph(e, flux, mass)) {
+        HIPCHK(hipGraphLaunch(e->row_exec, e->s));
+    } else {
         step_body_aligned(e, flux, mass);
         HIPCHK(hipGetLastError());
-        return 0;
     }
-    if (e->row_calls == GM_ROW_RECORD) {
-        if (e->row_exec) {
-            HIPCHK(hipGraphExecDestroy(e->row_exec));
-            e->row_exec = nullptr;
-        }
-        e->row_calls = 0;  // until the graph stands
-        hipGraph_t g;
-        HIPCHK(hipStreamBeginCapture(e->s, hipStreamCaptureModeThreadLocal));
-        step_body_aligned(e, flux, mass);
-        HIPCHK(hipStreamEndCapture(e->s, &g));
-        HIPCHK(hipGraphInstantiate(&e->row_exec, g, nullptr, nullptr, 0));
-        HIPCHK(hipGraphDestroy(g));
-    }
-    e->row_calls = GM_ROW_RECORD;
-    HIPCHK(hipGraphLaunch(e->row_exec, e->s));
     return 0;
 }
 

@@ -270,7 +270,9 @@ enum {
 
 /* SetupLevels (cF:115-264) + getStaticNodesAndElements/getStaticSubcycle:
  * allocates all level state on the current device and initialises it to
- * T_amb, S1 = 0.  `stream` is kept and used by every engine call. */
+ * T_amb, S1 = 0.  `stream` is kept and used by every engine call;
+ * the null stream takes no graph capture, which gm_engine_subcycle needs unless
+ * gm_engine_use_graph(e, 0). */
 int gm_engine_create(const gm_config* cfg, const gm_material* mat, void* stream,
                      gm_engine** out);
 int gm_engine_destroy(gm_engine* e);
@@ -365,7 +367,10 @@ int gm_multi_destroy(gm_multi* m);
  * return value _resetmask (cF:2394-2397: L3 nodes whose S2 went 0 -> 1) into
  * the GM_RESET_L3 field.  In the engine's own melt-time mode (the default,
  * see gm_engine_set_accum_mode) it also applies the single-step driver's
- * melt-time bookkeeping (go_melt.py:339-357) to the Level0 maps. */
+ * melt-time bookkeeping (go_melt.py:339-357) to the Level0 maps.  On
+ * node-aligned levels the step is recorded as a hipGraph at the eighth call
+ * with the same launches and replayed from then on; on a stream that takes no
+ * capture (the null stream) every call launches its kernels. */
 int gm_engine_step(gm_engine* e, const float* row_host);
 /* gm_engine_step by the kernels of levels that are not node-aligned, launched
  * one by one.  On node-aligned levels gm_engine_step takes merged kernels;
@@ -431,7 +436,8 @@ int gm_engine_minmax(gm_engine* e, float* minmax_host);
  * subcycle graph (advances the engine state).  Synchronous. */
 int gm_engine_time_kernel(gm_engine* e, int which, int iters, float* ms_per_launch);
 
-/* Enable/disable hipGraph capture of gm_engine_subcycle (default enabled). */
+/* Enable/disable hipGraph capture of gm_engine_subcycle and gm_engine_step
+ * (default enabled). */
 int gm_engine_use_graph(gm_engine* e, int enable);
 
 /* ------------------------------------------------------------------------ */

@@ -191,6 +191,35 @@ def test_single_step_routes_equal(tmp_path, deck):
             np.testing.assert_array_equal(a, b)
 
 
+def test_single_steps_on_the_null_stream(tmp_path):
+    """An engine on the null stream, which no graph can be recorded on: rows
+    past the call that records one elsewhere, and the state of an engine on a
+    stream of its own."""
+    import json
+    import _native as N
+    import computeFunctions as cf
+    import go_melt as G
+
+    class Null:
+        ptr = None
+
+        def sync(self):
+            N.sync(None)
+
+    states = []
+    for stream in (N.Stream(), Null()):
+        inp, g = W.tiny(n=(8, 8, 4), n2=2, n3=2, track=1.2)
+        with open(W.write_deck(inp, g, str(tmp_path / str(len(states))))) as fh, \
+                cf.engines_on_stream(stream):
+            run = G.TimeLoop(json.load(fh), quiet=True, write_outputs=False)
+        run.step_chunk(next(run.chunks()))
+        row = np.asarray(next(run.chunks())[0], np.float32)
+        for _ in range(20):
+            N.check(N.lib().gm_engine_step(run.eng.h, N.fptr(row)))
+        states.append(run.eng.save_state())
+    assert states[0] == states[1]
+
+
 def test_driver_vs_oracle_unaligned_windows(oracle, tmp_path):
     """L2 origin a quarter of an L1 spacing off the L1 nodes: the coarse
     overlap nodes are not fine nodes, so the engine takes the general
