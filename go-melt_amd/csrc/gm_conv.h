@@ -34,13 +34,32 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t conv_rsrc(const void* p, uint3
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, CONV_DW3);
 }
 
-// The marching convolution (gm_conv_march.hip).  conv_march_ok: whether it
-// takes these operands; the sums of every output run in the same order as
-// the other kernels', so both give the same bits.
-bool conv_march_ok(const ConvDims& c, const void* X, const void* Wk, const void* Y,
-                   const void* Ybf);
-void launch_conv_march(const ConvDims& c, const uint16_t* X, const uint16_t* Wk,
-                       const float* bias, int relu, float* Y, uint16_t* Ybf, hipStream_t s);
+// The marching convolution (gm_conv_march.hip): tile shape, cut of the volume
+// and estimated time of a launch.
+struct MarchCfg {
+    int xt, yw, nt, wv, s;
+    double lat;  // latency of a step, us (see march_plan)
+};
+// columns of a volume (x fastest, then y, z segments, batch) and output tiles
+struct TileGrid {
+    int nx, ny, nz, nt;
+    int zs;  // planes of a segment
+};
+struct MarchPlan {
+    MarchCfg g;
+    TileGrid tg;
+    int64_t blocks = 0;
+    size_t lds = 0;
+    double us = 0.0;
+};
+// whether the kernel takes these operands, and how.  Every output's sum runs
+// tap by tap, the channels inner, as in the unsplit k_conv_fwd32: the same
+// bits from both.
+bool conv_march_plan(const ConvDims& c, const void* X, const void* Wk, const void* Y,
+                     const void* Ybf, MarchPlan* p);
+void launch_conv_march(const MarchPlan& p, const ConvDims& c, const uint16_t* X,
+                       const uint16_t* Wk, const float* bias, int relu, float* Y, uint16_t* Ybf,
+                       hipStream_t s);
 
 // The weight gradient on transposing LDS reads (gm_conv_wgrad.hip).
 bool conv_wgrad_tr_ok(const ConvDims& c, const void* X, const void* dY);

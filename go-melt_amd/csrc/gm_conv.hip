@@ -16,8 +16,9 @@
 // here for unaligned or very large operands).
 //
 // The forward pass of inputs in multiples of 32 channels marches along z
-// (gm_conv_march.hip); the kernels here take the rest: 16-channel inputs, the
-// split sums of volumes with few tiles, unaligned or very large operands.
+// (gm_conv_march.hip) where its columns fill well; the kernels here take the
+// rest: 16-channel inputs, many small images, the split sums of volumes with
+// few tiles, unaligned or very large operands.
 //
 // Tiles: a block of 4 waves computes 64 x 64 outputs; each wave a 32 x 32
 // quarter as 2 x 2 MFMA tiles of 16 x 16 (k_conv_fwd32 on large volumes with
@@ -531,15 +532,55 @@ static void launch_plan(const FwdPlan& p, const ConvDims& c, const uint16_t* X,
     }
 }
 
+// Estimated time of k_conv_fwd32 on plan p, us: a chain of its 32-channel
+// sub-stages and their work over the CUs (64 x 64 or 128 x 32 tiles; 256 x 32
+// twice).  Fitted to 327 shapes of 200 to 6e5 voxels on one MI355X, 32 to 256
+// channels, within 10% (one standard deviation); march_plan's estimate is
+// within 15% there.
+static double fwd32_us(const FwdPlan& p, const ConvDims& c) {
+    const double n = 27.0 * (c.ci / 32), w = (double)p.grid.x * p.grid.y / 256.0;
+    if (c.co <= 32) return 5.5 + n * (0.5 + (p.small ? 0.2 : 0.5) * w);
+    return 5.5 + n * (0.34 + (p.small ? 0.15 : 0.18) * w);
+}
+
+// The marching kernel where it is estimated to be no slower: a column pads
+// small and ragged images to its tile, and k_conv_fwd32 packs their voxels.
+// Measured on one MI355X, us, k_conv_fwd32 and marching: 4096 images of one
+// voxel, 128 -> 128 45 and 616; 512 of 4x4x2 68 and 274; 8 of 17x17x17,
+// 256 -> 128 209 and 498; 16 of 18x18x16, 64 -> 64 80 and 78; 16 of 64x64x32,
+// 32 -> 32 446 and 160.  Over those 327 shapes the chosen kernel is the slower
+// one by more than 8% for ten (1.5 times at most).
+static bool march_chosen(const FwdPlan& p, const ConvDims& c, const void* X, const void* Wk,
+                         const void* Y, const void* Ybf, MarchPlan* m) {
+    return conv_march_plan(c, X, Wk, Y, Ybf, m) && (!p.fwd32 || m->us <= fwd32_us(p, c));
+}
+
+static void launch_unsplit(const FwdPlan& p, const ConvDims& c, const uint16_t* X,
+                           const uint16_t* Wk, const float* bias, int relu, float* Y,
+                           uint16_t* Ybf, hipStream_t s) {
+    MarchPlan m;
+    if (march_chosen(p, c, X, Wk, Y, Ybf, &m))
+        launch_conv_march(m, c, X, Wk, bias, relu, Y, Ybf, s);
+    else
+        launch_plan(p, c, X, Wk, bias, relu, Y, Ybf, nullptr, s);
+}
+
 void launch_conv_fwd(const int32_t* shape, const uint16_t* X, const uint16_t* Wk,
                      const float* bias, int relu, float* Y, uint16_t* Ybf, hipStream_t s) {
     const ConvDims c = dims(shape);
-    if (conv_march_ok(c, X, Wk, Y, Ybf)) {
-        launch_conv_march(c, X, Wk, bias, relu, Y, Ybf, s);
-        return;
-    }
     const bool al16 = (((uintptr_t)X | (uintptr_t)Wk) & 15) == 0;
-    launch_plan(plan_fwd(c, al16), c, X, Wk, bias, relu, Y, Ybf, nullptr, s);
+    launch_unsplit(plan_fwd(c, al16), c, X, Wk, bias, relu, Y, Ybf, s);
+}
+
+void conv_fwd_plan(const int32_t* shape, int32_t* out) {
+    const ConvDims c = dims(shape);
+    const FwdPlan p = plan_fwd(c, true);
+    MarchPlan m;
+    std::fill(out, out + 7, 0);
+    out[0] = p.fwd32;
+    if (!march_chosen(p, c, nullptr, nullptr, nullptr, nullptr, &m)) return;
+    const int32_t v[7] = {2, m.g.xt, m.g.yw, m.g.nt, m.g.wv, m.g.s, m.tg.nz};
+    std::copy(v, v + 7, out);
 }
 
 int64_t conv_fwd_split_bytes(const int32_t* shape) {
@@ -556,11 +597,10 @@ void launch_conv_fwd_ws(const int32_t* shape, const uint16_t* X, const uint16_t*
     const FwdPlan p = plan_fwd(c, al16);
     const bool split = p.fwd32 && p.splits > 1 && ws &&
                        ws_bytes >= (int64_t)p.splits * c.nvox * c.co * 4;
-    if (!split) {
-        launch_conv_fwd(shape, X, Wk, bias, relu, Y, Ybf, s);
-        return;
-    }
-    launch_plan(p, c, X, Wk, bias, relu, Y, Ybf, (float*)ws, s);
+    if (split)
+        launch_plan(p, c, X, Wk, bias, relu, Y, Ybf, (float*)ws, s);
+    else
+        launch_unsplit(p, c, X, Wk, bias, relu, Y, Ybf, s);
 }
 
 void launch_conv_wflip(int ci, int co, const uint16_t* Wk, uint16_t* Wt, hipStream_t s) {

@@ -38,12 +38,6 @@ struct ConvTile {
     static constexpr int PL = HX * HY;  // halo rows of a plane
 };
 
-// columns of a volume (x fastest, then y, z segments, batch) and output tiles
-struct TileGrid {
-    int nx, ny, nz, nt;
-    int zs;  // planes of a segment
-};
-
 extern __shared__ __align__(16) uint8_t conv_lds[];
 
 template <int XT, int YW, int NT, int WV, int S>
@@ -300,26 +294,12 @@ __global__ void __launch_bounds__(64 * WV, 2)
     }
 }
 
-// A launch of the kernel: its shape and how the columns are cut along z.
-struct MarchCfg {
-    int xt, yw, nt, wv, s;
-    double lat;  // latency of a step, us (see march_plan)
-};
-
 // All shapes the launcher instantiates.  s = 9: 32 input channels, weights
 // resident in LDS.
 static const MarchCfg kMarch[] = {
     {16, 2, 2, 8, 9, 0.02}, {16, 4, 1, 4, 9, 0.02}, {16, 2, 1, 4, 9, 0.02}, {8, 1, 2, 4, 9, 0.02},
     {8, 1, 1, 4, 9, 0.02},  {16, 2, 2, 8, 3, 0.13}, {16, 1, 4, 8, 1, 0.23}, {16, 1, 2, 8, 3, 0.10},
     {16, 1, 2, 4, 3, 0.16}, {16, 2, 1, 4, 3, 0.11}, {8, 1, 2, 4, 3, 0.16},  {8, 1, 1, 4, 3, 0.11}};
-
-struct MarchPlan {
-    MarchCfg g;
-    TileGrid tg;
-    int64_t blocks = 0;
-    size_t lds = 0;
-    double us = 0.0;
-};
 
 static const size_t kLds = 160 * 1024;
 
@@ -352,6 +332,7 @@ static bool march_plan(const ConvDims& c, MarchPlan* best) {
             p.tg.zs = (c.D + seg - 1) / seg;
             p.tg.nz = (c.D + p.tg.zs - 1) / p.tg.zs;
             p.blocks = (int64_t)c.nb * p.tg.nx * p.tg.ny * p.tg.nz * p.tg.nt;
+            if (p.blocks * 64 * g.wv >= (int64_t)1 << 32) continue;  // threads of a grid
             const double per_cu = std::min((double)res, ceil(p.blocks / 256.0));
             const double gens = ceil(p.blocks / (256.0 * per_cu));
             const int planes = std::min(p.tg.zs + 2, c.D);
@@ -361,18 +342,17 @@ static bool march_plan(const ConvDims& c, MarchPlan* best) {
             found = true;
         }
     }
-    return found && best->blocks < ((int64_t)1 << 31);
+    return found;
 }
 
 // 32-bit byte offsets within an image and the weights, 16-byte accesses
-bool conv_march_ok(const ConvDims& c, const void* X, const void* Wk, const void* Y,
-                   const void* Ybf) {
+bool conv_march_plan(const ConvDims& c, const void* X, const void* Wk, const void* Y,
+                     const void* Ybf, MarchPlan* p) {
     const int64_t lim = (int64_t)1 << 31;
-    MarchPlan p;
     return c.ci % 32 == 0 &&
            (((uintptr_t)X | (uintptr_t)Wk | (uintptr_t)Y) & 15) == 0 &&
            ((uintptr_t)Ybf & 7) == 0 && (int64_t)c.D * c.H * c.W * c.ci * 2 < lim &&
-           (int64_t)27 * c.ci * c.co * 2 < lim && march_plan(c, &p);
+           (int64_t)27 * c.ci * c.co * 2 < lim && march_plan(c, p);
 }
 
 template <int XT, int YW, int NT, int WV, int S>
@@ -380,16 +360,16 @@ static void launch_march(const MarchPlan& p, const ConvDims& c, const uint16_t* 
                          const uint16_t* Wk, const float* bias, int relu, float* Y,
                          uint16_t* Ybf, hipStream_t s) {
     const auto k = k_conv_march<XT, YW, NT, WV, S>;
-    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kLds);
+    if (p.lds > 64 * 1024)
+        (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)kLds);
     hipLaunchKernelGGL(k, dim3((unsigned)p.blocks), dim3(64 * WV), p.lds, s, c, p.tg, X, Wk, bias,
                        relu, Y, Ybf);
 }
 
-void launch_conv_march(const ConvDims& c, const uint16_t* X, const uint16_t* Wk,
-                       const float* bias, int relu, float* Y, uint16_t* Ybf, hipStream_t s) {
-    MarchPlan p;
-    if (!march_plan(c, &p)) return;
+void launch_conv_march(const MarchPlan& p, const ConvDims& c, const uint16_t* X,
+                       const uint16_t* Wk, const float* bias, int relu, float* Y, uint16_t* Ybf,
+                       hipStream_t s) {
     const MarchCfg& g = p.g;
 #define GM_MARCH(XT, YW, NT, WV, S)                                                    \
     if (g.xt == XT && g.yw == YW && g.nt == NT && g.wv == WV && g.s == S)              \

@@ -3067,6 +3067,14 @@ extern "C" int gm_conv3d_fwd(const int32_t* shape, const uint16_t* X, const uint
     return 0;
 }
 
+extern "C" int gm_conv3d_plan(int pass, const int32_t* shape, int32_t* out) {
+    if (!shape || !out) return fail("gm_conv3d_plan: null argument");
+    if (!conv_shape_ok(shape)) return fail("gm_conv3d_plan: bad shape");
+    if (pass != 0) return fail("gm_conv3d_plan: pass must be 0");
+    conv_fwd_plan(shape, out);
+    return 0;
+}
+
 extern "C" int gm_conv3d_fwd_ws_bytes(const int32_t* shape, int64_t* bytes) {
     if (!shape || !bytes) return fail("gm_conv3d_fwd_ws_bytes: null argument");
     if (!conv_shape_ok(shape)) return fail("gm_conv3d_fwd_ws_bytes: bad shape");

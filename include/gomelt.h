@@ -510,6 +510,13 @@ int gm_batch_jump_state(gm_batch* b, int i, const float* T0);
 int gm_conv3d_fwd(const int32_t* shape_host, const uint16_t* X, const uint16_t* Wk,
                   const float* bias, int relu, float* Y, uint16_t* Ybf, void* stream);
 
+/* Which kernel a call with 16-byte aligned operands and no workspace takes for
+ * a shape (host only).  pass 0: forward, or the gradient of the input with
+ * cin and cout exchanged.  out7: kernel (0 general, 1 pipelined tap by tap, 2
+ * marching along z), then for the marching kernel tile width, y rows a wave,
+ * output tiles, waves, weight steps a stage and z segments. */
+int gm_conv3d_plan(int pass, const int32_t* shape_host, int32_t* out7_host);
+
 /* The same forward pass with a caller's workspace: on volumes that give the
  * chip few output tiles (coarse U-Net levels, one window) the K sum (taps x
  * input channels) is split over blocks that write partial sums into ws,

@@ -89,10 +89,10 @@ def test_conv_gradients(S, shape):
     assert _rel(dW.cpu().numpy() - base, ref) < 1e-5
 
 
-# the marching kernel's edges: partial tiles in x, y and z, 8- and 16-wide
-# tiles, output counts off its tiles, one plane, one voxel, volumes cut into z
-# segments, channel stages up to the LDS limit and past it (352: the
-# tap-by-tap kernel), and few tiles (the split sum of the forward pass)
+# edges of the passes as a network calls them: partial tiles in x, y and z, 8-
+# and 16-wide tiles, output counts off the tiles, one plane, one voxel, 352
+# channels (the tap-by-tap kernel).  Most forward passes here have few tiles
+# and split their sum; MARCH_TILES holds the marching kernel's own edges
 MARCH = [(1, 3, 19, 33, 32, 48), (2, 5, 17, 8, 64, 96), (1, 33, 9, 40, 32, 80),
          (1, 1, 1, 1, 32, 16), (3, 1, 30, 23, 64, 32), (1, 7, 34, 17, 160, 32),
          (2, 4, 12, 20, 256, 64), (1, 2, 9, 16, 352, 16), (5, 17, 33, 40, 64, 64),
@@ -167,6 +167,53 @@ def test_conv_weight_gradient_edges(S, shape):
     torch.cuda.synchronize()
     assert _rel(dW.cpu().numpy() - base, ref) < 1e-5
     assert _rel(dWo.cpu().numpy(), ref) < 2e-5
+
+
+# every tile shape of the marching kernel, on one z segment and on several
+# (test_conv_plan checks that), with ragged x and y edges
+MARCH_TILES = [
+    (1, 1, 6, 5, 64, 16), (1, 4, 6, 7, 64, 16), (1, 1, 5, 5, 32, 16), (1, 4, 11, 5, 32, 16),
+    (15, 1, 39, 5, 160, 64), (11, 11, 10, 5, 64, 96), (11, 1, 25, 5, 32, 96),
+    (9, 4, 10, 5, 32, 64), (15, 1, 19, 10, 64, 96), (3, 8, 18, 9, 64, 64),
+    (16, 1, 10, 20, 64, 96), (11, 8, 5, 17, 64, 32), (11, 1, 41, 6, 160, 128),
+    (2, 12, 50, 35, 64, 64), (14, 1, 9, 10, 64, 96), (3, 4, 9, 10, 64, 96),
+    (9, 1, 10, 9, 32, 128), (6, 4, 9, 9, 32, 48), (10, 1, 59, 9, 64, 128),
+    (3, 35, 57, 9, 64, 32), (15, 1, 33, 9, 32, 128), (4, 15, 17, 10, 32, 96),
+    (13, 1, 35, 9, 32, 64), (3, 16, 9, 10, 32, 48)]
+
+
+@pytest.mark.parametrize("shape", MARCH_TILES)
+def test_conv_march_tiles(S, shape):
+    """The marching kernel without a workspace: FP32 output within 1e-5 of the
+    oracle's max (FP32 sums of exact bf16 products), the bf16 outputs (with
+    and without the FP32 one) its rounding, and the bits of the tap-by-tap
+    kernel, which an output off 16 bytes takes."""
+    import ctypes
+    import torch
+    import _native as N
+    from oracle import conv_oracle as CO
+    nb, D, H, W, ci, co = shape
+    rng = np.random.default_rng(17 + sum(shape))
+    X = CO.bf16_round(rng.standard_normal((nb, D, H, W, ci)).astype(np.float32))
+    Wk = CO.bf16_round((0.2 * rng.standard_normal((27, co, ci))).astype(np.float32))
+    b = rng.standard_normal(co).astype(np.float32)
+    Xd, Wd, bd = _dev_bf16(X), _dev_bf16(Wk), torch.from_numpy(b).cuda()
+    out = torch.full((nb * D * H * W * co + 2,), -7.0, device="cuda")
+    Y = torch.empty((nb, D, H, W, co), device="cuda")
+    Yb, Yo = (torch.empty(Y.shape, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    p = lambda t, o=0: ctypes.c_void_p(t.data_ptr() + o)  # noqa: E731
+    sh, L = (ctypes.c_int32 * 6)(*shape), N.lib()
+    N.check(L.gm_conv3d_fwd(sh, p(Xd), p(Wd), p(bd), 1, p(Y), p(Yb), None))
+    N.check(L.gm_conv3d_fwd_bf16(sh, p(Xd), p(Wd), p(bd), 1, p(Yo), None, 0, None))
+    N.check(L.gm_conv3d_fwd(sh, p(Xd), p(Wd), p(bd), 1, p(out, 8), None, None))
+    torch.cuda.synchronize()
+    Yn = Y.cpu().numpy()
+    assert _rel(Yn, np.maximum(CO.conv3d(X, Wk, b), 0)) < 1e-5
+    np.testing.assert_array_equal(Yb.float().cpu().numpy(), CO.bf16_round(Yn))
+    np.testing.assert_array_equal(Yo.float().cpu().numpy(), CO.bf16_round(Yn))
+    out = out.cpu().numpy()
+    np.testing.assert_array_equal(out[2:], Yn.reshape(-1))
+    assert (out[:2] == -7.0).all()
 
 
 def test_two_layer_training_gradients(S):

@@ -241,10 +241,11 @@ def test_layer_output_reads_fp32(S):
 
 
 @pytest.mark.parametrize("shape,ci,co", [((1, 4, 8, 8), 128, 128), ((1, 3, 5, 7), 48, 80),
-                                         ((2, 8, 16, 16), 32, 64), ((1, 4, 6, 10), 16, 32)])
+                                         ((2, 8, 16, 16), 32, 64), ((1, 4, 6, 10), 16, 32),
+                                         ((4, 9, 40, 47), 32, 32), ((5, 17, 33, 40), 64, 64)])
 def test_conv_bf16_output_only(S, shape, ci, co):
-    """want_f32=False (split K sum, general, marching and 16-channel kernels)
-    gives the bf16 output of the full call."""
+    """want_f32=False (split K sum, general, 16-channel and, on the last two,
+    marching kernels) gives the bf16 output of the full call."""
     import torch
     gen = torch.Generator().manual_seed(ci)
     X = torch.randn(shape + (ci,), generator=gen).bfloat16().cuda()
