@@ -62,8 +62,20 @@ void launch_conv_march(const MarchPlan& p, const ConvDims& c, const uint16_t* X,
                        hipStream_t s);
 
 // The weight gradient on transposing LDS reads (gm_conv_wgrad.hip).
-bool conv_wgrad_tr_ok(const ConvDims& c, const void* X, const void* dY);
-void launch_conv_wgrad_tr(const ConvDims& c, const uint16_t* X, const uint16_t* dY, float* dW,
-                          hipStream_t s);
+struct WgGrid {
+    int nx, ny, nz, zs;  // columns per axis, z segments of zs planes
+    int units;           // nb * nx * ny * nz
+};
+struct WgTrPlan {
+    int xt;     // column width
+    bool wide;  // 32 inputs a block
+    WgGrid g;
+    int gx;     // blocks a channel tile
+    double us;  // estimated time
+};
+// whether the kernel takes these operands, and how
+bool conv_wgrad_tr_plan(const ConvDims& c, const void* X, const void* dY, WgTrPlan* p);
+void launch_conv_wgrad_tr(const WgTrPlan& p, const ConvDims& c, const uint16_t* X,
+                          const uint16_t* dY, float* dW, hipStream_t s);
 
 }  // namespace gm

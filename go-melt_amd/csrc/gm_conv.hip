@@ -12,8 +12,8 @@
 // Wk[tap][o][i] for the forward pass and, with the flipped and transposed
 // weights Wk'[tap][i][o] = Wk[26-tap][o][i], for the gradient of the input.
 // The weight gradient dWk[tap][o][i] = sum_vox dY[vox][o] X[vox+s(tap)][i] is
-// a second kernel that reduces over voxels (gm_conv_wgrad.hip; k_conv_wgrad
-// here for unaligned or very large operands).
+// a second kernel that reduces over voxels (gm_conv_wgrad.hip; the tap-by-tap
+// ones here for many small images and for unaligned or very large operands).
 //
 // The forward pass of inputs in multiples of 32 channels marches along z
 // (gm_conv_march.hip) where its columns fill well; the kernels here take the
@@ -25,6 +25,8 @@
 // up to 32 outputs: waves of 64 voxels x 32 outputs); K advances through LDS one tap and
 // 32 input channels at a time (k_conv_fwd32, software-pipelined) or, for 16
 // input channels, 16 at a time (k_conv_fwd).
+
+#include <math.h>
 
 #include <algorithm>
 
@@ -467,6 +469,182 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(ConvDims c, const uint16_t* 
             }
 }
 
+// The same for cin and cout multiples of 32 (8 channels per 16-byte load), for
+// volumes that k_conv_wgrad_tr's columns would pad: stages of 32 voxels staged voxel-major ([vox][channel], 16-byte LDS
+// writes, no transpose), the next stage's loads in flight during the MFMAs;
+// a lane's fragment (4 consecutive voxels of one channel) is 4 LDS reads.
+// Tiles of OT outputs x 4096 / OT inputs: 64 x 64 (waves 2 x 2), or 32 x 128
+// (waves along the inputs) so that a 32-output layer fills whole tiles.
+template <int OT>
+__global__ void __launch_bounds__(256) k_conv_wgrad32(ConvDims c, const uint16_t* __restrict__ X,
+                                                      const uint16_t* __restrict__ dY, int vsplit,
+                                                      float* __restrict__ dW) {
+    constexpr int IT = 4096 / OT;  // inputs per tile
+    constexpr int NX = IT / 64;    // X loads per thread and stage
+    __shared__ uint16_t sA[32][OT + 8];  // [vox][o]
+    __shared__ uint16_t sB[32][IT + 8];  // [vox][i]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int o0 = blockIdx.x * OT, i0 = blockIdx.y * IT;
+    const int tap = blockIdx.z % 27, part = blockIdx.z / 27;
+    const int64_t per = (c.nvox + vsplit - 1) / vsplit;
+    const int64_t vbeg = (int64_t)part * per;
+    const int64_t vend = vbeg + per < c.nvox ? vbeg + per : c.nvox;
+    const int wm = OT == 64 ? (wave & 1) * 32 : 0, wn = OT == 64 ? (wave >> 1) * 32 : wave * 32;
+    v4f acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    // staging: 16-byte chunks (8 channels) of the stage's 32 voxels, chunk q
+    // = voxel q / (T/8), channels (q % (T/8)) * 8 of the T-wide tile: dY has
+    // 4 OT chunks (threads below 4 OT), the shifted X 4 IT (NX per thread)
+    const int sva = tid / (OT / 8), sca = (tid % (OT / 8)) * 8;
+    auto fetch = [&](int64_t vb, uint4& dv, uint4* xv) {
+        dv = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < 4 * OT && vb + sva < vend && o0 + sca < c.co)
+            dv = *(const uint4*)(dY + (vb + sva) * c.co + o0 + sca);
+#pragma unroll
+        for (int k = 0; k < NX; ++k) {
+            const int q = tid + 256 * k, svb = q / (IT / 8), scb = (q % (IT / 8)) * 8;
+            const int64_t v = vb + svb;
+            xv[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (v < vend && i0 + scb < c.ci) {
+                const int64_t vs = vox_shift(c, vox_decode(c, v), tap);
+                if (vs >= 0) xv[k] = *(const uint4*)(X + vs * c.ci + i0 + scb);
+            }
+        }
+    };
+    uint4 dv, xv[NX];
+    fetch(vbeg, dv, xv);
+    const int fi = lane & 15, fk = (lane >> 4) * 4;
+    for (int64_t vb = vbeg; vb < vend; vb += 32) {
+        __syncthreads();
+        if (tid < 4 * OT) *(uint4*)&sA[sva][sca] = dv;
+#pragma unroll
+        for (int k = 0; k < NX; ++k) {
+            const int q = tid + 256 * k;
+            *(uint4*)&sB[q / (IT / 8)][(q % (IT / 8)) * 8] = xv[k];
+        }
+        __syncthreads();
+        if (vb + 32 < vend) fetch(vb + 32, dv, xv);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            v4s fa[2], fb[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int ro = wm + t * 16 + fi, ri = wn + t * 16 + fi, k0 = ks * 16 + fk;
+                fa[t] = v4s{(short)sA[k0][ro], (short)sA[k0 + 1][ro], (short)sA[k0 + 2][ro],
+                            (short)sA[k0 + 3][ro]};
+                fb[t] = v4s{(short)sB[k0][ri], (short)sB[k0 + 1][ri], (short)sB[k0 + 2][ri],
+                            (short)sB[k0 + 3][ri]};
+            }
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[a], fb[b], acc[a][b],
+                                                                          0, 0, 0);
+        }
+    }
+    const int dj = lane & 15, di = (lane >> 4) * 4;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int o = o0 + wm + a * 16 + di + r;
+                const int i = i0 + wn + b * 16 + dj;
+                if (o < c.co && i < c.ci)
+                    atomicAdd(dW + ((int64_t)tap * c.co + o) * c.ci + i, acc[a][b][r]);
+            }
+}
+
+// Weight gradient for cout = CO and cin = CI, each 16 or 32 (the
+// full-resolution layers): each wave computes the whole CO x CI tile of one
+// tap over its own quarter of a 128-voxel stage (no idle half tiles), and
+// adds it with FP32 atomics.
+template <int CO, int CI>
+__global__ void __launch_bounds__(256) k_conv_wgrad32x(ConvDims c, const uint16_t* __restrict__ X,
+                                                       const uint16_t* __restrict__ dY,
+                                                       int vsplit, float* __restrict__ dW) {
+    constexpr int NA = CO / 16;           // MFMA tiles along cout
+    constexpr int NB = CI / 16;           // MFMA tiles along cin
+    __shared__ uint16_t sA[128][CO + 8];  // [vox][o]
+    __shared__ uint16_t sB[128][CI + 8];  // [vox][i]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tap = blockIdx.z % 27, part = blockIdx.z / 27;
+    const int64_t per = (c.nvox + vsplit - 1) / vsplit;
+    const int64_t vbeg = (int64_t)part * per;
+    const int64_t vend = vbeg + per < c.nvox ? vbeg + per : c.nvox;
+    v4f acc[NA][NB];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    // staging: 16 bytes (8 channels) of voxels t/4 and t/4 + 64, channels (t%4)*8
+    const int sv = tid >> 2, sc = (tid & 3) * 8;
+    auto fetch = [&](int64_t vb, uint4* dv, uint4* xv) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int64_t v = vb + sv + 64 * q;
+            dv[q] = make_uint4(0u, 0u, 0u, 0u);
+            xv[q] = make_uint4(0u, 0u, 0u, 0u);
+            if (v < vend) {
+                if (sc < CO) dv[q] = *(const uint4*)(dY + v * CO + sc);
+                const int64_t vs = vox_shift(c, vox_decode(c, v), tap);
+                if (vs >= 0 && sc < CI) xv[q] = *(const uint4*)(X + vs * CI + sc);
+            }
+        }
+    };
+    uint4 dv[2], xv[2];
+    fetch(vbeg, dv, xv);
+    const int fi = lane & 15, fk = (lane >> 4) * 4;
+    const int kw = wave * 32;  // this wave's voxels of the stage
+    for (int64_t vb = vbeg; vb < vend; vb += 128) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if (sc < CO) *(uint4*)&sA[sv + 64 * q][sc] = dv[q];
+            if (sc < CI) *(uint4*)&sB[sv + 64 * q][sc] = xv[q];
+        }
+        __syncthreads();
+        if (vb + 128 < vend) fetch(vb + 128, dv, xv);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int k0 = kw + ks * 16 + fk;
+            v4s fa[NA], fb[NB];
+#pragma unroll
+            for (int t = 0; t < NA; ++t) {
+                const int r = t * 16 + fi;
+                fa[t] = v4s{(short)sA[k0][r], (short)sA[k0 + 1][r], (short)sA[k0 + 2][r],
+                            (short)sA[k0 + 3][r]};
+            }
+#pragma unroll
+            for (int t = 0; t < NB; ++t) {
+                const int r = t * 16 + fi;
+                fb[t] = v4s{(short)sB[k0][r], (short)sB[k0 + 1][r], (short)sB[k0 + 2][r],
+                            (short)sB[k0 + 3][r]};
+            }
+#pragma unroll
+            for (int a = 0; a < NA; ++a)
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[a], fb[b], acc[a][b],
+                                                                          0, 0, 0);
+        }
+    }
+    const int dj = lane & 15, di = (lane >> 4) * 4;
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                atomicAdd(dW + ((int64_t)tap * CO + a * 16 + di + r) * CI + b * 16 + dj,
+                          acc[a][b][r]);
+}
+
 // Adam on FP32 master weights, with the bf16 copy the kernels read
 __global__ void k_adam(float* __restrict__ w, uint16_t* __restrict__ wbf,
                        const float* __restrict__ g, float* __restrict__ m,
@@ -609,18 +787,97 @@ void launch_conv_wflip(int ci, int co, const uint16_t* Wk, uint16_t* Wt, hipStre
                        Wk, Wt);
 }
 
+// The tap-by-tap weight gradients: blocks of one tap x a tile of channels x a
+// part of the voxels, `stage` voxels at a time.
+struct WgTapPlan {
+    int kernel = 0;  // 0 k_conv_wgrad, 1 k_conv_wgrad32<64>, 2 <32>, 3 k_conv_wgrad32x
+    int vsplit = 1;
+    dim3 grid;
+    double us = 0.0;  // estimated time
+};
+
+// Estimate: a chain of a block's stages and the stages of all blocks over the
+// CUs, fitted per kernel to 40 to 200 shapes of 200 to 6e5 voxels on one
+// MI355X (within 8%, k_conv_wgrad32x 16%, one standard deviation).
+static WgTapPlan plan_wgrad_tap(const ConvDims& c, bool al16) {
+    WgTapPlan p;
+    // about 1024 voxels per block, at most 2048 parts (grid z = 27 * parts);
+    // 4096 for 32 x 32 channels from 2^18 voxels on (each block adds its
+    // partial tile to dW with FP32 atomics: 163 us instead of 219 on 524288
+    // voxels; the other kernels were 2-6% slower with longer parts)
+    const bool long_parts = c.nvox >= ((int64_t)1 << 18) && c.ci == 32 && c.co == 32;
+    const int64_t per = long_parts ? 4096 : 1024;
+    p.vsplit = (int)std::min<int64_t>((c.nvox + per - 1) / per, 2048);
+    p.grid = dim3((unsigned)((c.co + 63) / 64), (unsigned)((c.ci + 63) / 64),
+                  (unsigned)(27 * p.vsplit));
+    int stage = 16;
+    double t0 = 8.5, chain = 0.5, work = 0.145;
+    if (al16 && (c.co == 32 || c.co == 16) && (c.ci == 32 || c.ci == 16)) {
+        p.kernel = 3;
+        p.grid.x = p.grid.y = 1;
+        stage = 128;
+        t0 = 6.6, chain = 0.32, work = 0.16 + 0.36 * (c.ci * c.co / 1024.0);
+    } else if (al16 && c.ci % 32 == 0 && c.co == 32) {
+        p.kernel = 2;
+        p.grid = dim3(1, (unsigned)((c.ci + 127) / 128), p.grid.z);
+        stage = 32;
+        t0 = 8.0, chain = 0.57, work = 0.28;
+    } else if (al16 && c.ci % 32 == 0 && c.co % 32 == 0) {
+        p.kernel = 1;
+        stage = 32;
+        t0 = 5.0, chain = 0.475, work = 0.195;
+    }
+    const double n = std::ceil(std::ceil((double)c.nvox / p.vsplit) / stage);
+    p.us = t0 + n * (chain + work * (double)p.grid.x * p.grid.y * p.grid.z / 256.0);
+    return p;
+}
+
+// k_conv_wgrad_tr where it is estimated to be no slower: its columns pad small
+// images, and every pass over a channel tile walks them.  Measured on one
+// MI355X, us, tap by tap and columns: 4096 images of one voxel, 128 x 128
+// channels 30 and 983; 512 of 4x4x2 61 and 259; 16 windows of 64x64x32, 32 x 32
+// 573 and 191.  Over 419 shapes the chosen kernel is the slower one by more
+// than 8% for seven (1.4 times at most).
+static bool wgrad_tr_chosen(const WgTapPlan& p, const ConvDims& c, const void* X, const void* dY,
+                            WgTrPlan* t) {
+    return conv_wgrad_tr_plan(c, X, dY, t) && t->us <= p.us;
+}
+
 void launch_conv_wgrad(const int32_t* shape, const uint16_t* X, const uint16_t* dY, float* dW,
                        hipStream_t s) {
     const ConvDims c = dims(shape);
-    if (conv_wgrad_tr_ok(c, X, dY)) {
-        launch_conv_wgrad_tr(c, X, dY, dW, s);
+    const WgTapPlan p = plan_wgrad_tap(c, (((uintptr_t)X | (uintptr_t)dY) & 15) == 0);
+    WgTrPlan t;
+    if (wgrad_tr_chosen(p, c, X, dY, &t)) {
+        launch_conv_wgrad_tr(t, c, X, dY, dW, s);
         return;
     }
-    // about 1024 voxels per block, at most 2048 parts (grid z = 27 * parts)
-    const int vsplit = (int)std::min<int64_t>((c.nvox + 1023) / 1024, 2048);
-    const dim3 grid((unsigned)((c.co + 63) / 64), (unsigned)((c.ci + 63) / 64),
-                    (unsigned)(27 * vsplit));
-    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, s, c, X, dY, vsplit, dW);
+    const dim3 g = p.grid, b(256);
+    if (p.kernel == 3 && c.co == 32 && c.ci == 32)
+        hipLaunchKernelGGL((k_conv_wgrad32x<32, 32>), g, b, 0, s, c, X, dY, p.vsplit, dW);
+    else if (p.kernel == 3 && c.co == 32)
+        hipLaunchKernelGGL((k_conv_wgrad32x<32, 16>), g, b, 0, s, c, X, dY, p.vsplit, dW);
+    else if (p.kernel == 3 && c.ci == 32)
+        hipLaunchKernelGGL((k_conv_wgrad32x<16, 32>), g, b, 0, s, c, X, dY, p.vsplit, dW);
+    else if (p.kernel == 3)
+        hipLaunchKernelGGL((k_conv_wgrad32x<16, 16>), g, b, 0, s, c, X, dY, p.vsplit, dW);
+    else if (p.kernel == 2)
+        hipLaunchKernelGGL(k_conv_wgrad32<32>, g, b, 0, s, c, X, dY, p.vsplit, dW);
+    else if (p.kernel == 1)
+        hipLaunchKernelGGL(k_conv_wgrad32<64>, g, b, 0, s, c, X, dY, p.vsplit, dW);
+    else
+        hipLaunchKernelGGL(k_conv_wgrad, g, b, 0, s, c, X, dY, p.vsplit, dW);
+}
+
+void conv_wgrad_plan(const int32_t* shape, int32_t* out) {
+    const ConvDims c = dims(shape);
+    const WgTapPlan p = plan_wgrad_tap(c, true);
+    WgTrPlan t;
+    std::fill(out, out + 7, 0);
+    out[0] = p.kernel ? 1 : 0;
+    if (!wgrad_tr_chosen(p, c, nullptr, nullptr, &t)) return;
+    const int32_t v[7] = {2, t.xt, t.wide ? 2 : 1, 0, 0, 0, t.g.nz};
+    std::copy(v, v + 7, out);
 }
 
 void launch_adam(float* w, uint16_t* wbf, const float* g, float* m, float* v, int64_t n, float lr,

@@ -3070,8 +3070,9 @@ extern "C" int gm_conv3d_fwd(const int32_t* shape, const uint16_t* X, const uint
 extern "C" int gm_conv3d_plan(int pass, const int32_t* shape, int32_t* out) {
     if (!shape || !out) return fail("gm_conv3d_plan: null argument");
     if (!conv_shape_ok(shape)) return fail("gm_conv3d_plan: bad shape");
-    if (pass != 0) return fail("gm_conv3d_plan: pass must be 0");
-    conv_fwd_plan(shape, out);
+    if (pass != 0 && pass != 1) return fail("gm_conv3d_plan: pass must be 0 or 1");
+    if (pass == 0) conv_fwd_plan(shape, out);
+    else conv_wgrad_plan(shape, out);
     return 0;
 }
 

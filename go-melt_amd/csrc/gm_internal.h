@@ -254,6 +254,7 @@ void launch_conv_fwd_ws(const int32_t* shape, const uint16_t* X, const uint16_t*
                         const float* bias, int relu, float* Y, uint16_t* Ybf, void* ws,
                         int64_t ws_bytes, hipStream_t s);
 void conv_fwd_plan(const int32_t* shape, int32_t* out7);
+void conv_wgrad_plan(const int32_t* shape, int32_t* out7);
 void launch_conv_wflip(int ci, int co, const uint16_t* Wk, uint16_t* Wt, hipStream_t s);
 void launch_conv_wgrad(const int32_t* shape, const uint16_t* X, const uint16_t* dY, float* dW,
                        hipStream_t s);

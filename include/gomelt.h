@@ -512,9 +512,10 @@ int gm_conv3d_fwd(const int32_t* shape_host, const uint16_t* X, const uint16_t* 
 
 /* Which kernel a call with 16-byte aligned operands and no workspace takes for
  * a shape (host only).  pass 0: forward, or the gradient of the input with
- * cin and cout exchanged.  out7: kernel (0 general, 1 pipelined tap by tap, 2
- * marching along z), then for the marching kernel tile width, y rows a wave,
- * output tiles, waves, weight steps a stage and z segments. */
+ * cin and cout exchanged; 1: weight gradient.  out7: kernel (0 general, 1 tap
+ * by tap on 16-byte loads, 2 marching along z), then for the marching kernels
+ * tile width, y rows a wave, output tiles, waves, weight steps a stage and z
+ * segments (pass 1: tile width, input tiles, three zeros and z segments). */
 int gm_conv3d_plan(int pass, const int32_t* shape_host, int32_t* out7_host);
 
 /* The same forward pass with a caller's workspace: on volumes that give the

@@ -5,7 +5,7 @@ import os
 import pytest
 
 import _native as N
-from test_gpu_conv import MARCH_TILES
+from test_gpu_conv import MARCH_TILES, WGRAD_TAPS, WGRAD_TILES
 
 
 def _plan(shape, kind=0):
@@ -41,3 +41,22 @@ def test_march_tiles_cover_the_kernel():
     ((16, 4, 8, 8, 128, 128), 2), ((1, 32, 64, 64, 32, 32), 2)])
 def test_forward_kernel_by_shape(shape, kernel):
     assert _plan(shape)[0] == kernel
+
+
+def test_weight_gradient_shapes_cover_the_kernels():
+    seen = set()
+    for s in WGRAD_TILES:
+        kernel, xt, it, _, _, _, nz = _plan(s, 1)
+        assert kernel == 2 and s[3] % xt and s[2] % (64 // xt), s
+        seen.add((xt, it, nz > 1))
+    assert seen == {(xt, it, many) for xt in (8, 16) for it in (1, 2) for many in (False, True)}
+    assert [_plan(s, 1)[0] for s in WGRAD_TAPS] == [1, 1, 1, 1, 1, 1, 0]
+
+
+@pytest.mark.parametrize("shape,kernel", [
+    ((4096, 1, 1, 1, 128, 128), 1), ((2048, 2, 2, 2, 256, 128), 1), ((512, 4, 4, 4, 192, 64), 1),
+    ((864, 9, 1, 1, 48, 256), 0), ((1, 130, 512, 512, 32, 32), 1), ((3, 13, 27, 35, 48, 80), 2),
+    ((16, 32, 64, 64, 32, 32), 2), ((16, 32, 64, 64, 96, 32), 2), ((16, 16, 32, 32, 64, 64), 2),
+    ((16, 8, 16, 16, 128, 128), 2), ((16, 4, 8, 8, 128, 128), 2)])
+def test_weight_gradient_kernel_by_shape(shape, kernel):
+    assert _plan(shape, 1)[0] == kernel

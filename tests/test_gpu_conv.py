@@ -132,6 +132,61 @@ def test_conv_march_edges(S, shape):
     assert _rel(dX.cpu().numpy(), CO.conv3d_bwd_data(dY, Wk)) < 1e-5
 
 
+# the weight gradient's column kernel on every tile shape, on one z segment and
+# on several, with ragged columns; then the tap-by-tap ones on many small
+# images (32 and 16 channels, 32 outputs, multiples of 32, others), the number
+# of voxels off their stages (test_conv_plan checks the kernels)
+WGRAD_TILES = [(1, 1, 14, 38, 16, 16), (1, 9, 13, 18, 48, 16), (7, 1, 17, 17, 32, 64),
+               (2, 9, 17, 18, 128, 32), (1, 1, 5, 25, 48, 16), (1, 9, 5, 27, 16, 48),
+               (3, 1, 9, 17, 96, 80), (5, 9, 9, 17, 32, 80)]
+WGRAD_TAPS = [(300, 1, 1, 1, 32, 32), (201, 2, 1, 1, 32, 16), (601, 1, 2, 2, 16, 32),
+              (901, 1, 2, 1, 16, 16), (901, 2, 1, 2, 96, 32), (131, 2, 2, 1, 64, 96),
+              (701, 1, 1, 2, 48, 80)]
+
+
+@pytest.mark.parametrize("shape", WGRAD_TILES + WGRAD_TAPS)
+def test_conv_weight_gradient_kernels(S, shape):
+    """Added to what dW holds: 1e-5 of the max against the oracle (FP32 sums
+    of exact bf16 products)."""
+    import torch
+    from oracle import conv_oracle as CO
+    nb, D, H, W, ci, co = shape
+    rng = np.random.default_rng(19 + sum(shape))
+    X = CO.bf16_round(rng.standard_normal((nb, D, H, W, ci)).astype(np.float32))
+    dY = CO.bf16_round(rng.standard_normal((nb, D, H, W, co)).astype(np.float32))
+    base = rng.standard_normal((27, co, ci)).astype(np.float32)
+    dW = torch.from_numpy(base.copy()).cuda()
+    S.conv3d_bwd_weight(_dev_bf16(X), _dev_bf16(dY), dW)
+    torch.cuda.synchronize()
+    assert _rel(dW.cpu().numpy() - base, CO.conv3d_bwd_weight(X, dY)) < 1e-5
+
+
+def test_conv_weight_gradient_large_image(S):
+    """An image of more than 2^31 bytes: gradients at a few voxels, the first
+    and last and those around byte 2^31 among them, against their own sums."""
+    import torch
+    D, H, W, ci, co = 130, 512, 512, 32, 16
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    X = torch.randn((1, D, H, W, ci), generator=gen, device="cuda", dtype=torch.bfloat16)
+    assert X.numel() * 2 > 2 ** 31
+    dY = torch.zeros((1, D, H, W, co), dtype=torch.bfloat16, device="cuda")
+    edge = 2 ** 31 // (2 * ci)
+    v = torch.cat([torch.tensor([0, edge - 1, edge, D * H * W - 1]),
+                   torch.randint(0, D * H * W, (300,), generator=torch.Generator().manual_seed(3))]
+                  ).unique().cuda()
+    g = torch.randn((len(v), co), generator=gen, device="cuda").bfloat16()
+    dY.view(-1, co)[v] = g
+    dW = torch.zeros((27, co, ci), device="cuda")
+    S.conv3d_bwd_weight(X, dY, dW)
+    z, y, x = v // (H * W), v // W % H, v % W
+    for tap in range(27):
+        zz, yy, xx = z + tap // 9 - 1, y + tap // 3 % 3 - 1, x + tap % 3 - 1
+        ok = (zz >= 0) & (zz < D) & (yy >= 0) & (yy < H) & (xx >= 0) & (xx < W)
+        rows = X.view(-1, ci)[((zz * H + yy) * W + xx)[ok]].double()
+        ref = (g[ok].double().t() @ rows).cpu().numpy()
+        assert _rel(dW[tap].cpu().numpy(), ref) < 1e-5, tap
+
+
 # the weight gradient's edges: partial 16 x 4 and 8 x 8 columns, segments of
 # one plane and cut volumes, an odd number of columns, channel tiles off 32,
 # one voxel
