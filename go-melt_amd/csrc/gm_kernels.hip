@@ -1607,9 +1607,14 @@ __global__ void __launch_bounds__(256) k_source_tables(GmPair p, const GmStepDes
 void launch_source_tables(const GmPair& p, const GmStepDesc* d, const DevMat& m, int row0,
                           int npos, int use_rows, const float* rows_dev, float* G, int nmax,
                           hipStream_t s) {
-    const int n = npos * 3 * nmax * SRC_L;
-    hipLaunchKernelGGL(k_source_tables, dim3((n + 255) / 256), dim3(256), 0, s, p, d, m, row0,
-                       npos, use_rows, rows_dev, G, nmax);
+    // a launch takes the positions whose threads (and entries) count in 30 bits
+    const int64_t most = std::max<int64_t>(1, ((int64_t)1 << 30) / (3 * SRC_L * (int64_t)nmax));
+    for (int64_t k = 0; k < npos; k += most) {
+        const int np = (int)std::min<int64_t>(most, npos - k);
+        const int n = np * 3 * nmax * SRC_L;
+        hipLaunchKernelGGL(k_source_tables, dim3((n + 255) / 256), dim3(256), 0, s, p, d, m,
+                           row0 + (int)k, np, use_rows, rows_dev, G + k * 3 * nmax, nmax);
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -119,6 +119,31 @@ def test_level_source(cf, oracle, pair):
     assert _rel(a, b) < 5e-6
 
 
+def test_level_source_many_positions(cf, oracle):
+    """50,000 positions on 1000 coarse elements (2.4e9 lanes of source
+    factors) of which the last three have power: three positions' source,
+    scaled by their share."""
+    import ctypes as C
+    import _native as N
+    _, p, _ = _deck(oracle, n=(4, 4, 2))
+    gc = N.gm_grid.make([1001, 3, 3], [0.0, 0.0, -0.04], [0.02] * 3)
+    gf = N.gm_grid.make([2001, 5, 5], [0.0, 0.0, -0.04], [0.01] * 3)
+    rows = np.zeros((50000, 7), np.float32)
+    rows[:, 0], rows[:, 1] = 5.0, 0.02
+    rows[-3:, 0], rows[-3:, 6] = (4.0, 9.0, 15.0), (100.0, 200.0, 300.0)
+
+    def source(r):
+        out = N.DeviceArray(gc.nn())
+        N.check(N.lib().gm_level_source(C.byref(gc), C.byref(gf), C.byref(cf._material(p)),
+                                        N.fptr(r), len(r), out.ptr, None))
+        return out.numpy().astype(np.float64)
+
+    few = source(rows[-3:].copy())
+    # three FP32 terms and their scale
+    assert _rel(source(rows) * (len(rows) / 3.0), few) < 1e-6
+    assert few.max() > 0
+
+
 def test_conv_rad(cf, oracle):
     _, p, L = _deck(oracle, n=(10, 9, 5), props={"emissivity": 0.4, "evaporation_coefficient": 0.82})
     rng = np.random.default_rng(3)
