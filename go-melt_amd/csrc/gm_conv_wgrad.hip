@@ -20,7 +20,7 @@ namespace gm {
 // at one dx feeds the three dz taps.  Rows are 96 bytes apart: the 32-byte
 // pieces of four consecutive rows hit distinct banks.  Positions of a tile
 // past the volume read zero rows for both operands.  After each column segment
-// (1024 voxels or fewer) the group adds its sums to the block's in LDS, which
+// (32 planes, 2048 voxels, or fewer) the group adds its sums to the block's in LDS, which
 // go to dW with FP32 atomics once at the end: short serial sums, and few
 // atomics.
 // ---------------------------------------------------------------------------
