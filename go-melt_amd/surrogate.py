@@ -46,10 +46,14 @@ def conv3d(X, Wk, bias=None, relu=False, want_bf16=True, want_f32=True):
     co = Wk.shape[1]
     if Wk.shape != (27, co, X.shape[4]):
         raise ValueError("Wk must be (27, cout, cin)")
-    out = X.shape[:4] + (co,)
-    Y = torch.empty(out, dtype=torch.float32, device=X.device) if want_f32 else None
-    Yb = torch.empty(out, dtype=torch.bfloat16, device=X.device) \
-        if want_bf16 or not want_f32 else None
+    # empty_like costs the host half of what empty does (1.1 us of 19 a small call)
+    out = dict(size=X.shape[:4] + (co,), device=X.device)
+    Y = torch.empty(dtype=torch.float32, **out) if want_f32 else None
+    Yb = None
+    if not want_f32:
+        Yb = torch.empty(dtype=torch.bfloat16, **out)
+    elif want_bf16:
+        Yb = torch.empty_like(Y, dtype=torch.bfloat16)
     if bias is not None:
         _check(bias, torch.float32, "bias")
     shape = _shape(X, co)
